@@ -104,6 +104,38 @@ int64_t column_split_tiles(int64_t n_tiles, int nct, int cus) {
     return ceil_div(left * 2 * nct, 8) <= fit64 ? t_split : 0;
 }
 
+int conv_split_pick(int64_t n, int ci, int co, int ncg) {
+    if (n <= 0 || co % (64 * ncg) != 0) return 0;
+    const int64_t cus = cu_count(), nkc = ci / HB_KC, tiles = ceil_div(n, HB_M);
+    // The kernels' times in us (fits to single convs of 1.2K-117K voxels, 64-1024 channels): a round
+    // of units costs so much per 16-channel slice, plus a fixed part (the large-grid kernel's tiles
+    // are pipelined and pay it once; a thin last round costs it 5.6 a slice, column_split_tiles).
+    const int64_t big = tiles * (co % 128 == 0 ? co / 128 : co / 64);
+    const double per = co % 128 == 0 ? 9.3 : 4.6;
+    int64_t whole = ceil_div(big, cus);
+    double base = 9.0;
+    if (ncg == 1 && co % 128 == 0 && column_split_tiles(tiles, co / 128, (int)cus) > 0) {
+        whole -= 1;
+        base += 5.6 * (double)nkc;
+    }
+    double best = 0.95 * (base + per * (double)(whole * nkc));   // (a margin: the split must be worth it)
+    int pick = 0;
+    const int64_t full = n / HB_M, rem = n % HB_M;
+    const int64_t last = rem ? std::min<int64_t>(4, ceil_div(rem, 32)) : 0;   // row groups of the last tile
+    for (int rgw = 4 / ncg; rgw >= 1; rgw /= 2) {
+        const int64_t units = (full * (4 / rgw) + ceil_div(last, rgw)) * (co / (64 * ncg));
+        const int w = rgw * ncg;
+        const int64_t rounds = ceil_div(units, cus);
+        const double slice = w == 4 ? 4.6 : w == 2 ? (rounds > 1 ? 2.45 : 2.2) : (rounds > 1 ? 1.6 : 1.45);
+        const double cost = 4.0 + (double)rounds * (6.0 + slice * (double)nkc);
+        if (cost < best) {
+            best = cost;
+            pick = rgw;
+        }
+    }
+    return pick;
+}
+
 int halo_conv_launch(int fdt, int odt, const void* feats, int64_t n, int ci, const int32_t* nbr,
                      const void* plan, const void* weight, const float* bias, int co, void* out,
                      hipStream_t s, OctantScatter osc, SkipAdd skip, PadRow pad, RowNorm ln, TileRange tr) {
@@ -139,6 +171,13 @@ int halo_conv_launch(int fdt, int odt, const void* feats, int64_t n, int ci, con
         set_error("MFMA conv: n * ci * 2 = %lld bytes of features exceed the 4 GiB the LDS-staged "
                   "kernel addresses", (long long)(n * ci * 2));
         return TSP_ERR_UNSUPPORTED;
+    }
+    // grids that leave most of the chip idle, or a costly last round, take the small-grid kernel
+    const int ncg = (ln.w && co == 128) || (osc.norm_silu && osc.cout == 128) ? 2 : 1;
+    if (const int rgw = conv_split_pick(n, ci, co, ncg)) {
+        auto* split = fdt == TSP_BF16 ? (rgw == 1 ? split_launch_bf16_1 : rgw == 2 ? split_launch_bf16_2 : split_launch_bf16_4)
+                                      : (rgw == 1 ? split_launch_f16_1 : rgw == 2 ? split_launch_f16_2 : split_launch_f16_4);
+        return split(odt, planned, feats, n, ci, nbr, plan, weight, bias, co, out, s, osc, skip, pad, ln, tr, ncg);
     }
     auto* fn64 = fdt == TSP_BF16 ? halo_launch_bf16_64 : halo_launch_f16_64;
     auto* fn = bn128 ? (fdt == TSP_BF16 ? halo_launch_bf16_128 : halo_launch_f16_128) : fn64;

@@ -1135,5 +1135,13 @@ int halo_launch_bf16_128(TSP_HALO_LAUNCH_ARGS);
 int halo_launch_bf16_64(TSP_HALO_LAUNCH_ARGS);
 int halo_launch_f16_128(TSP_HALO_LAUNCH_ARGS);
 int halo_launch_f16_64(TSP_HALO_LAUNCH_ARGS);
+// The small-grid kernel (conv_split_kernel.hpp), one translation unit per dtype and row groups of a
+// unit; ncg = 2 for the stores that need 128 whole channels (conv_split_{bf16,f16}_{1,2,4}.hip).
+int split_launch_bf16_1(TSP_HALO_LAUNCH_ARGS, int ncg);
+int split_launch_bf16_2(TSP_HALO_LAUNCH_ARGS, int ncg);
+int split_launch_bf16_4(TSP_HALO_LAUNCH_ARGS, int ncg);
+int split_launch_f16_1(TSP_HALO_LAUNCH_ARGS, int ncg);
+int split_launch_f16_2(TSP_HALO_LAUNCH_ARGS, int ncg);
+int split_launch_f16_4(TSP_HALO_LAUNCH_ARGS, int ncg);
 
 }  // namespace tsp

@@ -147,6 +147,12 @@ struct TileRange {
 // 64-channel grid takes in one: returns that t, or 0 for one launch (cus: compute units).
 int64_t column_split_tiles(int64_t n_tiles, int nct, int cus);
 
+// How many of a tile's four row groups a unit of the small-grid kernel takes (1, 2 or 4) for n
+// voxels, or 0 where the large-grid kernel serves better; ncg: 64-channel groups of a unit (2 for
+// the stores that need 128 whole channels, else 1). A rule on sizes alone: with and without a plan,
+// and over any tiles of it, a conv takes the same kernel and sums in the same order.
+int conv_split_pick(int64_t n, int ci, int co, int ncg);
+
 // tr (planned only): the plan's tiles to run, all of them by default; a narrower range runs in one
 // launch of its units.
 int halo_conv_launch(int fdt, int odt, const void* feats, int64_t n, int ci, const int32_t* nbr,

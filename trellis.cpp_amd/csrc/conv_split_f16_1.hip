@@ -1,0 +1,14 @@
+// Small-grid MFMA conv: the f16 instantiations with 1 row group a unit.
+#include "conv_split_kernel.hpp"
+
+namespace tsp {
+
+int split_launch_f16_1(TSP_HALO_LAUNCH_ARGS, int ncg) {
+    if (ncg == 2)
+        return split_launch<false, 1, 2>(odt, planned, feats, n, ci, nbr, plan, weight, bias, co, out, s, osc, skip,
+                                       pad, ln, tr);
+    return split_launch<false, 1, 1>(odt, planned, feats, n, ci, nbr, plan, weight, bias, co, out, s, osc, skip, pad,
+                                   ln, tr);
+}
+
+}  // namespace tsp
