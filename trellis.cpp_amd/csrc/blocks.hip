@@ -206,6 +206,31 @@ __global__ void k_f32_to(const float* __restrict__ x, int64_t n, void* __restric
     }
 }
 
+// The rounding pass for 16-bit types on 16-byte aligned buffers: 8 elements a thread and step, two
+// 16-byte loads and one 16-byte store. Bound by memory: 6 bytes an element at the rate of a copy
+// (600 K x 128, 460 MB: 74 us, 6.2 TB/s; one element a thread and step took 120 us, with a quarter
+// of the bytes in flight). The last n % 8 elements are the last thread's.
+template <int DT, bool SILU>
+__global__ __launch_bounds__(256) void k_f32_to16_vec(const float* __restrict__ x, int64_t n, uint16_t* __restrict__ y) {
+    const int64_t n8 = n / 8;
+    auto f = [](float v) {
+        if constexpr (SILU) v = v / (1.0f + expf(-v));
+        return v;
+    };
+    for (int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x; e < n8; e += (int64_t)gridDim.x * 256) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(x + 8 * e), b = *reinterpret_cast<const f32x4_t*>(x + 8 * e + 4);
+        const float v[8] = {f(a[0]), f(a[1]), f(a[2]), f(a[3]), f(b[0]), f(b[1]), f(b[2]), f(b[3])};
+        uint32_t w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            w[k] = DT == TSP_BF16 ? f32x2_to_bf16x2_bits(v[2 * k], v[2 * k + 1])
+                                  : f32_to_f16_bits(v[2 * k]) | ((uint32_t)f32_to_f16_bits(v[2 * k + 1]) << 16);
+        *reinterpret_cast<u32x4_t*>(y + 8 * e) = u32x4_t{w[0], w[1], w[2], w[3]};
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 255)
+        for (int64_t e = 8 * n8; e < n; ++e) st<DT>(y, e, f(x[e]));
+}
+
 template <int XDT>
 __global__ void k_add_to(float* __restrict__ y, const void* __restrict__ x, int64_t n) {
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n;
@@ -228,6 +253,19 @@ inline unsigned grid_for(int64_t total) {
 
 int f32_to(const float* x, int64_t n, void* y, int ydt, bool silu, hipStream_t s) {
     if (n <= 0) return TSP_OK;
+    if (ydt != TSP_F32 && !(reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(y) % 16)) {
+        const dim3 g(grid_for(ceil_div(n, 8))), b(256);
+        auto* y16 = static_cast<uint16_t*>(y);
+        if (ydt == TSP_F16) {
+            if (silu) hipLaunchKernelGGL((k_f32_to16_vec<TSP_F16, true>), g, b, 0, s, x, n, y16);
+            else hipLaunchKernelGGL((k_f32_to16_vec<TSP_F16, false>), g, b, 0, s, x, n, y16);
+        } else {
+            if (silu) hipLaunchKernelGGL((k_f32_to16_vec<TSP_BF16, true>), g, b, 0, s, x, n, y16);
+            else hipLaunchKernelGGL((k_f32_to16_vec<TSP_BF16, false>), g, b, 0, s, x, n, y16);
+        }
+        TSP_CHECK_LAUNCH();
+        return TSP_OK;
+    }
     const dim3 g(grid_for(n)), b(256);
 #define TSP_F32_TO(DT)                                                                     \
     if (silu) hipLaunchKernelGGL((k_f32_to<DT, true>), g, b, 0, s, x, n, y);               \
