@@ -156,6 +156,10 @@ int halo_conv_launch(int fdt, int odt, const void* feats, int64_t n, int ci, con
                   "(co=%d cout=%d)", bn128 ? 64 : 32, co, osc.cout);
         return TSP_ERR_UNSUPPORTED;
     }
+    if (osc.oct_tiles && (osc.cout % 128 != 0 || osc.blocks || !all_tiles)) {
+        set_error("MFMA conv: an octant plan needs cout %% 128 == 0 (cout=%d) and is run whole", osc.cout);
+        return TSP_ERR_UNSUPPORTED;
+    }
     if (osc.norm_silu && (!bn128 || (osc.cout != 64 && osc.cout != 128) || odt != fdt)) {
         set_error("MFMA conv: octant stores with the child norm need cout = 64 or 128, co %% 128 == 0 and "
                   "output in the feature type (co=%d cout=%d)", co, osc.cout);
@@ -184,7 +188,7 @@ int halo_conv_launch(int fdt, int odt, const void* feats, int64_t n, int ci, con
     // With a plan, whole rounds of 128-channel units and the tiles left over as 64-channel units
     // (kernels where either width runs: not the row norms, which need whole rows in a workgroup)
     if (!all_tiles) return fn(odt, planned, feats, n, ci, nbr, plan, weight, bias, co, out, s, osc, skip, pad, ln, tr);
-    if (planned && bn128 && !ln.w && !osc.norm_silu) {
+    if (planned && bn128 && !ln.w && !osc.norm_silu && !osc.oct_tiles) {
         const int64_t t_split = column_split_tiles(ceil_div(n, HB_M), co / 128, cu_count());
         if (t_split > 0) {
             if (int st = fn(odt, planned, feats, n, ci, nbr, plan, weight, bias, co, out, s, osc, skip, pad, ln,

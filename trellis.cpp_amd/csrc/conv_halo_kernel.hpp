@@ -108,7 +108,13 @@ __device__ __forceinline__ void conv_grid(
     // The workgroups of an XCD walk its range with a stride of their count (a multiple of
     // n_ctiles, so a workgroup keeps one column tile): with a stored plan the grid is one
     // workgroup per CU, otherwise one workgroup per pair.
-    const int64_t total = n_tiles * n_ctiles;
+    int64_t total = n_tiles * n_ctiles;
+    if constexpr (EPI == 1 || EPI == 5) {
+        if (osc.oct_tiles) {   // an octant plan: its tile count is known on the device only
+            total = min<int64_t>(n_tiles, *osc.oct_tiles) * n_ctiles;
+            per_xcd = (total + 7) / 8;
+        }
+    }
     const int xcd = (int)(blockIdx.x % 8);
     const int64_t xlo = xcd * per_xcd, xhi = xlo + per_xcd < total ? xlo + per_xcd : total;
     conv_tiles<BF16, BN, ODT, PLANNED, RB, CB, PD, SP, STG, EPI>(
@@ -221,6 +227,14 @@ __device__ __forceinline__ void conv_tiles(
     // with an octant scatter, the wave's channels lie in octant oct, from column ocol of a child
     const int oct = EPI == 1 || EPI == 4 || EPI == 5 ? c0 / osc.cout : 0;
     const int ocol = EPI == 1 || EPI == 4 || EPI == 5 ? c0 - oct * osc.cout : 0;
+    // the plan's tile of unit lin: on an octant plan, tile k of the unit's octant is 8 k + octant
+    const int unit_oct = (EPI == 1 || EPI == 5) && osc.oct_tiles ? (int)(lin0 % n_ctiles) * BN / osc.cout : -1;
+    auto plan_tile = [&](int64_t lin) -> int64_t {
+        if constexpr (EPI == 1 || EPI == 5) {
+            if (unit_oct >= 0) return lin / n_ctiles * 8 + unit_oct;
+        }
+        return lin / n_ctiles;
+    };
     const int nkc = ci / HB_KC;
     // The reference's absent taps read the padding row 0 * feats[0] (submconv_pad,
     // sparse.cpp:81-85), zeros here. Where row 0 holds an Inf or a NaN that row is NaN in those
@@ -749,7 +763,7 @@ __device__ __forceinline__ void conv_tiles(
         asm volatile("" : "+v"(lane), "+v"(r32), "+v"(g), "+v"(rg), "+v"(plane));
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) asm volatile("" : "+v"(boff[cb]));
-        const int64_t tile = lin / n_ctiles;
+        const int64_t tile = plan_tile(lin);
         const int64_t row0 = tile * HB_M;
         if (!pre) {
             // ---- tile plan: slot table in LDS, rows of this thread's slice pieces in registers
@@ -903,7 +917,7 @@ __device__ __forceinline__ void conv_tiles(
                 // the next tile of this workgroup (this one again after the last: its loads are
                 // then only unused copies)
                 const int64_t nlin = lin + stride < xhi ? lin + stride : lin;
-                const int64_t ntile = nlin / n_ctiles;
+                const int64_t ntile = plan_tile(nlin);
                 const int32_t* nhdr = plan.hdr + ntile * 4;
                 const int32_t nH = nhdr[0], ndirect = nhdr[1];
                 int32_t nrow[PIECES];
@@ -1012,7 +1026,7 @@ template <bool BF16, int BN, int ODT, bool PLANNED>
 int launch(const void* feats, int64_t n, int ci, const int32_t* nbr, const void* plan,
            const void* weight, const float* bias, int co, void* out, hipStream_t s, OctantScatter osc,
            SkipAdd skip, PadRow pad, RowNorm ln, TileRange tr) {
-    const int64_t all_tiles = ceil_div(n, HB_M);
+    const int64_t all_tiles = osc.oct_tiles ? osc.oct_cap : ceil_div(n, HB_M);   // (an octant plan: of each octant)
     // a stored plan's tiles [t0, t0 + n_tiles): its per-tile arrays (and the octant block words)
     // start at tile t0, and the kernel's tile indices count from there
     const int64_t t0 = PLANNED ? tr.t0 : 0;
@@ -1028,7 +1042,7 @@ int launch(const void* feats, int64_t n, int ci, const int32_t* nbr, const void*
     const int64_t per_xcd = ceil_div(total, 8);
     PlanView pv{};
     if (plan) {
-        pv = carve_plan(const_cast<void*>(plan), all_tiles);
+        pv = carve_plan(const_cast<void*>(plan), osc.oct_tiles ? 8 * all_tiles : all_tiles);
         pv.hdr += t0 * 4;
         pv.rowof += t0 * HB_SLOTS;
         pv.slots += t0 * HB_SLOT_TABLE;

@@ -91,7 +91,29 @@ struct OctantScatter {
     // parent of 32-row block b of that row group keeps octant o. The MFMAs of a block whose
     // parents keep none of a wave's octant are skipped: those outputs are never stored.
     const uint32_t* blocks = nullptr;
+    // Optional, an octant plan (octant_plan_build; its tiles are the `plan` argument then): *oct_tiles
+    // tiles of each octant, oct_cap at most, tile k of octant o at 8 k + o; cout % 128 == 0. Every
+    // MFMA then works for a row that is stored, where with `blocks` a block of 32 parents is rarely
+    // without one that keeps the octant. The sums are the same bits.
+    const int32_t* oct_tiles = nullptr;
+    int oct_cap = 0;
 };
+
+// An octant plan: for each octant, the parents that keep it as tiles of `rows` parents in the order
+// of the plan's walk, with their own distinct rows, slots and act bits. The octants' tiles take
+// turns, so that the units running together on an XCD share feature rows: with an octant's tiles
+// in a row instead, each XCD streamed every feature row (256 -> 128 at 60 K parents: 1100 us).
+struct OctantPlan {
+    int rows = 0;         // parents of a tile (a multiple of 32 up to HB_M)
+    int cap = 0;          // tiles of an octant, at most
+    size_t plan_bytes = 0, member_bytes = 0, count_bytes = 0;
+};
+// Whether conv1 of n parents and m children (cin -> 8 cout) takes an octant plan, and its sizes.
+bool octant_plan_spec(int64_t n, int64_t m, int cin, int cout, OctantPlan& op);
+// Builds it from the parents' stored plan, table and mask: tiles into oplan (op.plan_bytes); members
+// and counts are scratch; *oct_tiles: the tiles of the octant that has most.
+int octant_plan_build(const OctantPlan& op, const void* plan, int64_t n, const int32_t* nbr, const uint8_t* mask,
+                      void* oplan, int32_t* members, int32_t* counts, int32_t* oct_tiles, hipStream_t s);
 
 // The words OctantScatter::blocks reads, for a stored plan of n parents and their mask [8 n]:
 // out [n_tiles * 4].

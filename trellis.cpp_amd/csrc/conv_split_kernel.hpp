@@ -56,6 +56,13 @@ __global__ __launch_bounds__(512, 1) void k_conv_split(
     // Each XCD takes a contiguous range of units. Units in column-tile-major order keep an XCD on
     // few weight columns, in tile-major order on few feature rows: the caller picks by which is
     // larger, the weights or the features.
+    constexpr bool OCT = EPI == 1 || EPI == 4 || EPI == 5;
+    if constexpr (EPI == 1 || EPI == 5) {
+        if (osc.oct_tiles) {   // an octant plan: its tile count is known on the device only
+            n_tiles = min<int64_t>(n_tiles, *osc.oct_tiles);
+            per_xcd = (n_tiles * n_ctiles * RS + 7) / 8;
+        }
+    }
     const int64_t units = n_tiles * n_ctiles * RS;
     const int64_t u = (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (blockIdx.x / 8 >= per_xcd || u >= units) return;
@@ -71,6 +78,9 @@ __global__ __launch_bounds__(512, 1) void k_conv_split(
         const int k = (int)(u % ((int64_t)n_ctiles * RS));
         ct = k / RS;
         rsub = k % RS;
+    }
+    if constexpr (EPI == 1 || EPI == 5) {
+        if (osc.oct_tiles) tile = tile * 8 + ct * BN / osc.cout;   // tile k of octant o: 8 k + o
     }
     const int64_t row0 = tile * HB_M;
 
@@ -117,7 +127,7 @@ __global__ __launch_bounds__(512, 1) void k_conv_split(
         may_skip = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(weight) +
                                                       (size_t)kTaps * ci * co * 2) == 0u;
     uint32_t ob = 0xffffffffu;                       // octant stores: blocks that keep the wave's octant
-    const int oct = EPI == 1 || EPI == 4 || EPI == 5 ? c0 / osc.cout : 0;
+    const int oct = OCT ? c0 / osc.cout : 0;
     if constexpr (EPI == 1 || EPI == 4 || EPI == 5) {
         if (osc.blocks) {
             const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)osc.blocks[tile * 4 + rg]);
@@ -548,7 +558,7 @@ int split_launch(int odt, bool planned, const void* feats, int64_t n, int ci, co
                  SkipAdd skip, PadRow pad, RowNorm ln, TileRange tr) {
     constexpr int BN = 64 * NCG;
     constexpr int O16 = BF16 ? TSP_BF16 : TSP_F16;
-    const int64_t all_tiles = ceil_div(n, HB_M);
+    const int64_t all_tiles = osc.oct_tiles ? osc.oct_cap : ceil_div(n, HB_M);   // (an octant plan: of each octant)
     const int64_t t0 = planned ? tr.t0 : 0;
     const int64_t n_tiles = planned && tr.nt >= 0 ? tr.nt : all_tiles - t0;
     if (t0 < 0 || n_tiles < 0 || t0 + n_tiles > all_tiles) {
@@ -562,7 +572,7 @@ int split_launch(int odt, bool planned, const void* feats, int64_t n, int ci, co
     const bool ctile_major = n < (int64_t)kTaps * co;
     PlanView pv{};
     if (planned) {
-        pv = carve_plan(const_cast<void*>(plan), all_tiles);
+        pv = carve_plan(const_cast<void*>(plan), osc.oct_tiles ? 8 * all_tiles : all_tiles);
         pv.hdr += t0 * 4;
         pv.rowof += t0 * HB_SLOTS;
         pv.slots += t0 * HB_SLOT_TABLE;

@@ -605,6 +605,15 @@ __global__ __launch_bounds__(HB_PLAN_NT) __attribute__((amdgpu_waves_per_eu(6)))
     for (int t = 0; t < kTaps; ++t) sl[t * HB_M] = (uint16_t)(wsl[t >> 1] >> (16 * (t & 1)));
 }
 
+// The voxels of an octant plan's tiles: tile k of octant o is tile q = 8 k + o, its voxels
+// members[HB_M q ..], `rows` of them at most, of the octant's totals[o]; *tiles tiles an octant.
+struct OctantMembers {
+    const int32_t* members = nullptr;
+    const int32_t* tiles = nullptr;
+    const int32_t* totals = nullptr;
+    int rows = 0;
+};
+
 // Tiles ranked from the table's entries: tiles list[0 .. *list_n) (cell walk order when the grid is
 // in cell mode), or, without a list, tiles 0 .. n_tiles of consecutive rows. A workgroup takes
 // tiles blockIdx.x, + gridDim.x, ...
@@ -614,7 +623,7 @@ __global__ __launch_bounds__(HB_PLAN_NT) __attribute__((amdgpu_waves_per_eu(4)))
                                                            const GridHdr* __restrict__ hdr,
                                                            const int32_t* __restrict__ list,
                                                            const int32_t* __restrict__ list_n, int64_t n_tiles,
-                                                           PlanView plan) {
+                                                           PlanView plan, OctantMembers om) {
     static_assert(HB_PLAN_SCRATCH >= PL_ORDER_WORDS, "the order step fits the scratch");
     __shared__ __attribute__((aligned(16))) uint16_t sL[kTaps][4][32][4];
     __shared__ __attribute__((aligned(16))) int32_t sRowOf[HB_SLOTS];
@@ -625,11 +634,16 @@ __global__ __launch_bounds__(HB_PLAN_NT) __attribute__((amdgpu_waves_per_eu(4)))
     __shared__ uint32_t sAct[4 * HB_ACT_WORDS];
     const int tid = threadIdx.x;
     const bool walk = order != nullptr && hdr->mode == GRID_MODE_CELLS;
-    const int64_t count = list ? (int64_t)*list_n : n_tiles;
+    const int64_t count = list ? (int64_t)*list_n : om.members ? min<int64_t>(8 * (int64_t)*om.tiles, n_tiles) : n_tiles;
     for (int64_t k = blockIdx.x; k < count; k += gridDim.x) {
         const int64_t tile = list ? (int64_t)list[k] : k;
         const int64_t q = tile * HB_M + tid;
-        int64_t i[1] = {q < n ? (walk ? (int64_t)order[q] : q) : -1};
+        int64_t i[1];
+        if (om.members) {
+            i[0] = tid < om.rows && (tile >> 3) * om.rows + tid < om.totals[tile & 7] ? (int64_t)om.members[q] : -1;
+        } else {
+            i[0] = q < n ? (walk ? (int64_t)order[q] : q) : -1;
+        }
         int32_t nv[kTaps][1];
         load_entries<1>(nbr, n, i, nv);
         uint32_t taps = 0;
@@ -654,7 +668,163 @@ __global__ __launch_bounds__(HB_PLAN_NT) __attribute__((amdgpu_waves_per_eu(4)))
     }
 }
 
+// ---- octant plans ------------------------------------------------------------------------------
+// The octants a parent's mask bytes keep, a bit each.
+__device__ __forceinline__ uint32_t kept_octants(const uint8_t* __restrict__ mask, int32_t v) {
+    const uint64_t mw = *reinterpret_cast<const uint64_t*>(mask + 8 * (int64_t)v);
+    uint32_t kept = 0;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) kept |= (((mw >> (8 * o)) & 0xffull) != 0 ? 1u : 0u) << o;
+    return kept;
+}
+
+// counts[o n_tiles + tile] = the parents of plan tile `tile` that keep octant o.
+__global__ __launch_bounds__(HB_M) void k_octant_count(const int32_t* __restrict__ vox, int64_t n,
+                                                       const uint8_t* __restrict__ mask, int64_t n_tiles,
+                                                       int32_t* __restrict__ counts) {
+    __shared__ int sC[8];
+    const int tid = threadIdx.x;
+    if (tid < 8) sC[tid] = 0;
+    __syncthreads();
+    const int32_t v = vox[(int64_t)blockIdx.x * HB_M + tid];
+    const uint32_t kept = v >= 0 && v < n ? kept_octants(mask, v) : 0u;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+        const uint64_t b = __ballot((kept >> o) & 1u);
+        if ((tid & 63) == 0 && b) atomicAdd(&sC[o], __popcll(b));
+    }
+    __syncthreads();
+    if (tid < 8) counts[tid * n_tiles + blockIdx.x] = sC[tid];
+}
+
+// One workgroup, 128 threads an octant: the counts' exclusive prefixes over the tiles, in place; then
+// the octants' totals and the most tiles of one.
+__global__ __launch_bounds__(1024) void k_octant_scan(int64_t n_tiles, int rows, int32_t* __restrict__ counts,
+                                                      int32_t* __restrict__ totals, int32_t* __restrict__ oct_tiles) {
+    __shared__ int sS[1024];
+    __shared__ int sT[8];
+    const int tid = threadIdx.x, o = tid >> 7, t = tid & 127;
+    const int64_t chunk = (n_tiles + 127) / 128, b = t * chunk, e = min<int64_t>(n_tiles, b + chunk);
+    int32_t* c = counts + o * n_tiles;
+    int sum = 0;
+    for (int64_t k = b; k < e; ++k) sum += c[k];
+    sS[tid] = sum;
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int k = 0; k < 128; ++k) {
+        const int v = sS[(o << 7) + k];
+        before += k < t ? v : 0;
+        all += v;
+    }
+    for (int64_t k = b; k < e; ++k) {
+        const int v = c[k];
+        c[k] = before;
+        before += v;
+    }
+    if (t == 0) sT[o] = all;
+    __syncthreads();
+    if (tid == 0) {
+        int most = 0;
+        for (int k = 0; k < 8; ++k) {
+            totals[k] = sT[k];
+            most = max(most, sT[k]);
+        }
+        *oct_tiles = (most + rows - 1) / rows;
+    }
+}
+
+// Each kept (parent, octant) to its place: rank r of octant o is position r % rows of the octant's
+// tile r / rows. Ranks follow the plan's tiles and, inside a tile, the rows (a bitonic sort in LDS):
+// where an octant's tile ends inside a plan tile, that cuts the patch along an axis. In the plan's
+// own positions, grouped by corner taps, the cut is scattered over the patch: 1750-1870 distinct rows
+// a tile instead of 1440-1500 on bands, and 4-16 % of the tiles past HB_SLOTS.
+__global__ __launch_bounds__(HB_M) void k_octant_members(const int32_t* __restrict__ vox, int64_t n,
+                                                         const uint8_t* __restrict__ mask, int64_t n_tiles, int rows,
+                                                         int cap, const int32_t* __restrict__ counts,
+                                                         int32_t* __restrict__ members) {
+    __shared__ int sW[8][HB_M / 64];
+    __shared__ uint32_t sV[HB_M];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    sV[tid] = (uint32_t)vox[(int64_t)blockIdx.x * HB_M + tid];   // (-1, no voxel, sorts last)
+    __syncthreads();
+    for (int k = 2; k <= HB_M; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            const int u = tid ^ j;
+            if (u > tid) {
+                const uint32_t a = sV[tid], b = sV[u];
+                if ((a > b) == ((tid & k) == 0)) {
+                    sV[tid] = b;
+                    sV[u] = a;
+                }
+            }
+            __syncthreads();
+        }
+    const int32_t v = (int32_t)sV[tid];
+    const uint32_t kept = v >= 0 && v < n ? kept_octants(mask, v) : 0u;
+    int before[8];
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+        const uint64_t b = __ballot((kept >> o) & 1u);
+        before[o] = __popcll(b & ((1ull << lane) - 1ull));
+        if (lane == 0) sW[o][wave] = __popcll(b);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+        if (!((kept >> o) & 1u)) continue;
+        int r = counts[o * n_tiles + blockIdx.x] + before[o];
+        for (int w = 0; w < wave; ++w) r += sW[o][w];
+        if (r / rows < cap) members[((int64_t)(r / rows) * 8 + o) * HB_M + r % rows] = v;
+    }
+}
+
 }  // namespace
+
+bool octant_plan_spec(int64_t n, int64_t m, int cin, int cout, OctantPlan& op) {
+    // Half of the octants are kept on a surface band (m = 4.1 n), so the plan halves conv1; its build
+    // costs 40-60 us up to 100 K parents. Taken where conv1 is long enough to pay (150 us at the rate
+    // of the full conv), where it leaves out a fifth of the work at least, and where the kernel's
+    // 128-column tiles lie in one octant. The C2S block, us with and without: 60 K 256 -> 128 642 and
+    // 890; 12 K 512 -> 256 525 and 717; 33.5 K 1024 -> 512 4990 and 7260.
+    if (cout % 128 != 0 || n <= 0 || m <= 0) return false;
+    const double pay = conv_split_pick(n, cin, 8 * cout, cout == 128 ? 2 : 1) ? 7e8 : 4.3e8;   // (idle CUs: less to win)
+    if ((double)n * cin * cout < pay || 10 * m > 64 * n) return false;
+    // A tile's parents span rows / (m / 8n) voxels of the walk, which stage at most HB_SLOTS distinct
+    // rows: 1.4 rows a voxel on bands, up to 1.7.
+    const int64_t rows = std::min<int64_t>(HB_M, 1216 * m / (8 * n) / 32 * 32);
+    if (rows < 192) return false;
+    const int64_t cap = ceil_div(std::min(n, m), rows), tiles = ceil_div(n, HB_M);   // (every parent keeps an octant)
+    if (cap > INT32_MAX / 16) return false;
+    op.rows = (int)rows;
+    op.cap = (int)cap;
+    op.plan_bytes = plan_tile_bytes(8 * cap);
+    op.member_bytes = (size_t)cap * 8 * HB_M * 4;
+    op.count_bytes = ((size_t)tiles * 8 + 8) * 4;
+    return true;
+}
+
+int octant_plan_build(const OctantPlan& op, const void* plan, int64_t n, const int32_t* nbr, const uint8_t* mask,
+                      void* oplan, int32_t* members, int32_t* counts, int32_t* oct_tiles, hipStream_t s) {
+    const int64_t tiles = ceil_div(n, HB_M);
+    const PlanView pv = carve_plan(const_cast<void*>(plan), tiles);
+    int32_t* totals = counts + 8 * tiles;
+    hipLaunchKernelGGL(k_octant_count, dim3((unsigned)tiles), dim3(HB_M), 0, s, pv.vox, n, mask, tiles, counts);
+    TSP_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_octant_scan, dim3(1), dim3(1024), 0, s, tiles, op.rows, counts, totals, oct_tiles);
+    TSP_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_octant_members, dim3((unsigned)tiles), dim3(HB_M), 0, s, pv.vox, n, mask, tiles, op.rows,
+                       op.cap, counts, members);
+    TSP_CHECK_LAUNCH();
+    OctantMembers om;
+    om.members = members;
+    om.tiles = oct_tiles;
+    om.totals = totals;
+    om.rows = op.rows;
+    hipLaunchKernelGGL(k_plan_table, dim3((unsigned)std::min(8 * op.cap, 4096)), dim3(HB_PLAN_NT), 0, s, nbr, n, nullptr,
+                       nullptr, nullptr, nullptr, (int64_t)8 * op.cap, carve_plan(oplan, 8 * (int64_t)op.cap), om);
+    TSP_CHECK_LAUNCH();
+    return TSP_OK;
+}
 
 size_t halo_plan_bytes(int64_t n) {
     const int64_t n_tiles = std::max<int64_t>(1, ceil_div(n, HB_M));
@@ -690,7 +860,7 @@ static int plan_on_grid(const int32_t* nbr, const int32_t* coords, int64_t n, vo
     TSP_CHECK_LAUNCH();
     const unsigned grid = (unsigned)std::min<int64_t>(n_tiles, 512);
     hipLaunchKernelGGL(k_plan_table, dim3(grid), dim3(HB_PLAN_NT), 0, s, nbr, n, ps.order, gt.hdr, list, list_n,
-                       n_tiles, pv);
+                       n_tiles, pv, OctantMembers{});
     TSP_CHECK_LAUNCH();
     return TSP_OK;
 }
@@ -708,7 +878,7 @@ int halo_plan_build(const int32_t* nbr, const int32_t* coords, int64_t n, void* 
         return plan_on_grid(nbr, coords, n, plan, static_cast<const int32_t*>(ps.region), ps.tail, s, nullptr);
     }
     hipLaunchKernelGGL(k_plan_table, dim3((unsigned)n_tiles), dim3(HB_PLAN_NT), 0, s, nbr, n, nullptr, nullptr,
-                       nullptr, nullptr, n_tiles, carve_plan(plan, n_tiles));
+                       nullptr, nullptr, n_tiles, carve_plan(plan, n_tiles), OctantMembers{});
     TSP_CHECK_LAUNCH();
     return TSP_OK;
 }
