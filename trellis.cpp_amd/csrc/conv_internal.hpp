@@ -42,6 +42,11 @@ bool blaslt_eligible(int x_dtype, int weight_dtype, int out_dtype, int ci, int c
                      const void* w, const void* out);
 int blaslt_linear(const void* x, int xdt, int64_t n, int ci, const void* w, const float* bias,
                   int co, int act, const float* residual, void* out, int odt, hipStream_t s);
+// A linear layer of at most 16 outputs (linear_thin.hip): 16-bit x and weights of one dtype, Ci a
+// power of two from 32 to 512, 16-byte aligned x and weights, out f32 or that dtype. Returns
+// TSP_ERR_UNSUPPORTED (with no message) for anything else.
+int linear_thin_launch(int xdt, int wdt, int odt, const void* x, int64_t n, int ci, const void* w, const float* bias,
+                       int co, void* out, hipStream_t s);
 // The ConvNeXt MLP in one kernel (mlp.hip): y = x + b2 + W2 . silu(W0 . xn + b0) for 16-bit xn and
 // weights of one dtype dt, C = 128, the weights packed by mlp_pack (mlp_packed_bytes(c) bytes: W0
 // then W2 in MFMA operand order), 16-byte aligned xn and packed (mlp_fused_eligible). With y16
