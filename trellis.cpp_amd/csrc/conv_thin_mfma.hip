@@ -115,25 +115,32 @@ __global__ __launch_bounds__(TM_THREADS) void k_conv_thin_mfma(
     const int64_t per_xcd = (nchunks + 7) / 8;
     const int64_t xlo = (int64_t)(blockIdx.x % 8) * per_xcd;
     const int64_t xhi = xlo + per_xcd < nchunks ? xlo + per_xcd : nchunks;
-    for (int64_t chunk = xlo + (int64_t)(blockIdx.x / 8) * TM_WAVES + wave; chunk < xhi;
-         chunk += (int64_t)(gridDim.x / 8) * TM_WAVES) {
-        // table entries of every (block, step) first, then the rows they name: all loads of the
-        // chunk in flight together. Both go through buffer resources with 32-bit offsets (the
-        // launch checks that the table and the features span less than 2 GiB): an entry of a
-        // padding tap or a voxel past n is read out of range (0) and replaced by n, and the row of
-        // an absent tap is read out of range: zeros.
-        int32_t e[RB][NS];
+    // The table entries of a chunk's (block, step)s, all in flight together, and a chunk ahead of the
+    // rows they name: the next chunk's are read behind this chunk's rows, so that a chunk waits for
+    // one memory round trip and not for two. Entries and rows go through buffer resources with 32-bit
+    // offsets (the launch checks that the table and the features span less than 2 GiB): an entry of a
+    // padding tap or a voxel past n (or past the last chunk) is read out of range (0) and replaced by
+    // n, and the row of an absent tap is read out of range: zeros.
+    constexpr bool AHEAD = CI <= 16;   // (at 32 the 27 entries more cost a wave its place: 182 -> 260 us)
+    auto load_entries_of = [&](int64_t chunk, int32_t (&e)[RB][NS]) {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const int64_t i = chunk * CH + 16 * rb + v16;
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                const bool real = tap[s] < kTaps && i < n;
+                const bool real = tap[s] < kTaps && chunk < xhi && i < n;
                 const uint32_t off = real ? ((uint32_t)tap[s] * (uint32_t)n + (uint32_t)i) * 4u : tab_end;
                 const int32_t v = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rn, off, 0, 0);
                 e[rb][s] = real ? v : (int32_t)n;
             }
         }
+    };
+    const int64_t stride = (int64_t)(gridDim.x / 8) * TM_WAVES;
+    int64_t chunk = xlo + (int64_t)(blockIdx.x / 8) * TM_WAVES + wave;
+    int32_t e[RB][NS];
+    if constexpr (AHEAD) load_entries_of(chunk, e);
+    for (; chunk < xhi; chunk += stride) {
+        if constexpr (!AHEAD) load_entries_of(chunk, e);
         u32x4_t a[RB][NS];
         uint64_t absent_bits[RB];
 #pragma unroll
@@ -147,6 +154,10 @@ __global__ __launch_bounds__(TM_THREADS) void k_conv_thin_mfma(
                 // an absent real tap (the padding rows of k beyond 27 taps do not count)
                 absent_bits[rb] |= __ballot(!have && tap[s] < kTaps);
             }
+        }
+        if constexpr (AHEAD) {
+            load_entries_of(chunk + stride, e);
+            __builtin_amdgcn_sched_barrier(0);
         }
         f32x4_t acc[RB][NCB];
 #pragma unroll
@@ -210,12 +221,18 @@ __global__ __launch_bounds__(TM_THREADS) void k_conv_thin_mfma(
 template <bool BF16, int ODT, int CI, int NCB>
 int launch_tm(const void* feats, int64_t n, const int32_t* nbr, const void* weight, const float* bias, int co,
               void* out, hipStream_t s, PadRow pad) {
-    // 16-voxel blocks per chunk: two at Ci = 8, where a block's operands take 28 registers
-    constexpr int RB = CI == 8 ? 2 : 1;
+    // 16-voxel blocks per chunk: four at Ci = 8, where a block's operands take 28 registers
+    constexpr int RB = CI == 8 ? 4 : 1;
     const int64_t nchunks = ceil_div(n, 16 * RB);
-    // a multiple of 8 workgroups (one range per XCD), at most 4 a CU
+    // A multiple of 8 workgroups (one range per XCD), as many a CU as are resident together (their
+    // registers: two, or three at Ci = 16 with one column block): with more, an XCD's range is walked
+    // by workgroups that start late, and its L2 holds fewer of the rows they share. Us a conv on sets
+    // that are not in cache, against four a CU of two blocks with each chunk's entries read in turn:
+    // 1.69 M 8 -> 8 74 -> 70, 300 K 18.2 -> 13.7; 1.69 M 16 -> 16 127 -> 105; 1.69 M 32 -> 16
+    // 182 -> 174, 100 K 19 -> 16.
+    constexpr int PER_CU = CI == 16 && NCB == 1 ? 3 : 2;
     const int64_t blocks = std::max<int64_t>(
-        8, std::min<int64_t>(ceil_div(nchunks, TM_WAVES * 8) * 8, (int64_t)cu_count_tm() * 4 / 8 * 8));
+        8, std::min<int64_t>(ceil_div(nchunks, TM_WAVES * 8) * 8, (int64_t)cu_count_tm() * PER_CU / 8 * 8));
     hipLaunchKernelGGL((k_conv_thin_mfma<BF16, ODT, CI, NCB, RB>), dim3((unsigned)blocks),
                        dim3(TM_THREADS), 0, s, static_cast<const uint16_t*>(feats), n, nbr,
                        static_cast<const uint16_t*>(weight), bias, co,
