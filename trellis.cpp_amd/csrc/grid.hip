@@ -9,7 +9,6 @@ namespace tsp {
 namespace {
 
 constexpr int GB_NT = 256;        // threads of the grid-build workgroups
-constexpr int BBOX_PARTS = GRID_PARTS;   // workgroups of the bounding-box pass
 
 __device__ __forceinline__ int wave_min_i(int v) {
     for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
@@ -66,16 +65,15 @@ __global__ __launch_bounds__(GB_NT) void k_grid_bbox(const int32_t* __restrict__
 // Every workgroup reduces the bounding-box partials and sizes the directory (the same answer in
 // each; workgroup 0 writes the header), then the directory is cleared.
 __global__ __launch_bounds__(GB_NT) void k_grid_clear(const int32_t* __restrict__ parts, GridHdr* __restrict__ hdr,
-                                                      int32_t* __restrict__ dir, int64_t region_words) {
-    static_assert(BBOX_PARTS % GB_NT == 0, "whole partials per thread");
-    static_assert(BBOX_PARTS == GRID_PARTS, "the ascending flags fill their partials");
+                                                      int32_t* __restrict__ dir, int64_t region_words, int np) {
     __shared__ int sR[6][GB_NT / 64];
     __shared__ GridHdr sH;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 #pragma unroll
     for (int a = 0; a < 6; ++a) {
-        int v = parts[6 * tid + a];
-        for (int p = tid + GB_NT; p < BBOX_PARTS; p += GB_NT) {
+        int v = a < 3 ? INT32_MAX : -1;
+#pragma unroll 4
+        for (int p = tid; p < np; p += GB_NT) {
             const int u = parts[6 * p + a];
             v = a < 3 ? min(v, u) : max(v, u);
         }
@@ -83,7 +81,7 @@ __global__ __launch_bounds__(GB_NT) void k_grid_clear(const int32_t* __restrict_
         if (lane == 0) sR[a][wave] = r;
     }
     bool desc = false;
-    for (int p = tid; p < BBOX_PARTS; p += GB_NT) desc |= parts[6 * GRID_PARTS + p] == 0;
+    for (int p = tid; p < np; p += GB_NT) desc |= parts[6 * GRID_PARTS + p] == 0;
     const bool ascending = !__syncthreads_or(desc);
     if (tid == 0) {
         int lo[3], hi[3];
@@ -146,13 +144,13 @@ __global__ __launch_bounds__(GB_NT) void k_grid_mark(const int32_t* __restrict__
     }
 }
 
-// Occupied directory words of each of GRID_PARTS chunks into parts[].
+// Occupied directory words of each of np chunks into parts[].
 __global__ __launch_bounds__(GB_NT) void k_grid_scan(const GridHdr* __restrict__ hdr, const int32_t* __restrict__ dir,
-                                                     int32_t* __restrict__ parts) {
+                                                     int32_t* __restrict__ parts, int np) {
     __shared__ int sW[GB_NT / 64];
     if (hdr->mode != GRID_MODE_CELLS) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int64_t nw = hdr->dir_n, chunk = (nw + GRID_PARTS - 1) / GRID_PARTS;
+    const int64_t nw = hdr->dir_n, chunk = (nw + np - 1) / np;
     const int64_t b = blockIdx.x * chunk, e = min(nw, b + chunk);
     int c = 0;
     for (int64_t i = b + tid; i < e; i += GB_NT) c += dir[i] != 0;
@@ -166,7 +164,7 @@ __global__ __launch_bounds__(GB_NT) void k_grid_scan(const GridHdr* __restrict__
     }
 }
 
-// Every workgroup sums the GRID_PARTS partials for its own prefix and the block count, and
+// Every workgroup sums the np partials for its own prefix and the block count, and
 // decides whether the blocks fit the region and the caller's block_cap (the same answer in each;
 // workgroup 0 records it). Then: block
 // numbers into the directory (Morton order; cell_of, when given, gets each block's directory
@@ -174,8 +172,7 @@ __global__ __launch_bounds__(GB_NT) void k_grid_scan(const GridHdr* __restrict__
 // buckets cleared.
 __global__ __launch_bounds__(GB_NT) void k_grid_apply(GridHdr* __restrict__ hdr, int32_t* __restrict__ dir,
                                                       const int32_t* __restrict__ parts, HashView hash,
-                                                      int32_t* __restrict__ cell_of, int64_t block_cap) {
-    constexpr int PPT = GRID_PARTS / GB_NT;
+                                                      int32_t* __restrict__ cell_of, int64_t block_cap, int np) {
     __shared__ int sW[2][GB_NT / 64];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     bool cells = hdr->mode == GRID_MODE_CELLS;
@@ -183,9 +180,8 @@ __global__ __launch_bounds__(GB_NT) void k_grid_apply(GridHdr* __restrict__ hdr,
     int run = 0;
     if (cells) {
         int v = 0, before = 0;
-#pragma unroll
-        for (int k = 0; k < PPT; ++k) {
-            const int p = tid * PPT + k;
+#pragma unroll 4
+        for (int p = tid; p < np; p += GB_NT) {
             const int x = parts[p];
             if (p < (int)blockIdx.x) before += x;
             v += x;
@@ -213,7 +209,7 @@ __global__ __launch_bounds__(GB_NT) void k_grid_apply(GridHdr* __restrict__ hdr,
             w[s] = u32x4_t{0u, 0u, 0u, 0u};
         return;
     }
-    const int64_t nw = hdr->dir_n, chunk = (nw + GRID_PARTS - 1) / GRID_PARTS;
+    const int64_t nw = hdr->dir_n, chunk = (nw + np - 1) / np;
     const int64_t b = blockIdx.x * chunk, e = min(nw, b + chunk);
     for (int64_t r0 = b; r0 < e; r0 += GB_NT) {
         const int64_t i = r0 + tid;
@@ -304,18 +300,19 @@ int grid_build(const int32_t* coords, int64_t n, void* region, size_t region_byt
                int32_t* status, HashView hash, int32_t* cell_of, int64_t block_cap, hipStream_t s) {
     const GridTail gt = carve_grid_tail(tail);
     int32_t* dir = static_cast<int32_t*>(region);
+    const unsigned np = (unsigned)grid_parts(n);
     const unsigned nvb = (unsigned)std::max<int64_t>(1, ceil_div(n, GB_NT));
-    hipLaunchKernelGGL(k_grid_bbox, dim3(BBOX_PARTS), dim3(GB_NT), 0, s, coords, n, gt.parts, status);
+    hipLaunchKernelGGL(k_grid_bbox, dim3(np), dim3(GB_NT), 0, s, coords, n, gt.parts, status);
     TSP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_grid_clear, dim3(GRID_PARTS), dim3(GB_NT), 0, s, gt.parts, gt.hdr, dir,
-                       (int64_t)(region_bytes / 4));
+    hipLaunchKernelGGL(k_grid_clear, dim3(np), dim3(GB_NT), 0, s, gt.parts, gt.hdr, dir,
+                       (int64_t)(region_bytes / 4), (int)np);
     TSP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_grid_mark, dim3(nvb), dim3(GB_NT), 0, s, coords, n, gt.hdr, dir);
     TSP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_grid_scan, dim3(GRID_PARTS), dim3(GB_NT), 0, s, gt.hdr, dir, gt.parts);
+    hipLaunchKernelGGL(k_grid_scan, dim3(np), dim3(GB_NT), 0, s, gt.hdr, dir, gt.parts, (int)np);
     TSP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_grid_apply, dim3(GRID_PARTS), dim3(GB_NT), 0, s, gt.hdr, dir, gt.parts, hash, cell_of,
-                       block_cap);
+    hipLaunchKernelGGL(k_grid_apply, dim3(np), dim3(GB_NT), 0, s, gt.hdr, dir, gt.parts, hash, cell_of,
+                       block_cap, (int)np);
     TSP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_grid_insert, dim3(nvb), dim3(GB_NT), 0, s, coords, n, gt.hdr, dir, hash);
     TSP_CHECK_LAUNCH();

@@ -22,10 +22,18 @@
 namespace tsp {
 
 constexpr int32_t kCoordMax = (1 << 21) - 3;   // voxel coordinates in [0, kCoordMax]
-constexpr int GRID_PARTS = 1024;               // workgroups of the grid's scans
+constexpr int GRID_PARTS = 1024;               // workgroups of the grid's scans, at most
 constexpr int GRID_MAX_BITS = 10;              // directory of at most 2^30 cells
 constexpr size_t GRID_TAIL = 32768;            // bytes: header + GRID_PARTS * 7 partials
 constexpr int GRID_MODE_CELLS = 0, GRID_MODE_FALLBACK = 1;
+
+// The workgroups (and partials) of the scans for n voxels: one per 256 voxels, 64 at least. Each
+// workgroup reads every partial, so a small set's scans are short only with few of them (table and
+// plan of 15 K voxels 56.6 -> 52.7 us, of 1.5 K 52 -> 47, against 1024 always).
+inline int grid_parts(int64_t n) {
+    const int64_t p = ((n + 255) / 256 + 63) / 64 * 64;
+    return (int)(p < 64 ? 64 : p > GRID_PARTS ? GRID_PARTS : p);
+}
 
 struct GridHdr {
     int32_t mode;           // GRID_MODE_CELLS or GRID_MODE_FALLBACK

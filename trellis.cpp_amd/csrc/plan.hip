@@ -53,13 +53,13 @@ __device__ __forceinline__ uint64_t pack_xyz(int32_t x, int32_t y, int32_t z) {
 __global__ __launch_bounds__(WK_NT) void k_walk_count(const int32_t* __restrict__ coords, int64_t n,
                                                       const int32_t* __restrict__ dir, const GridHdr* __restrict__ hdr,
                                                       int32_t* __restrict__ counts, uint8_t* __restrict__ pres,
-                                                      int32_t* __restrict__ parts) {
+                                                      int32_t* __restrict__ parts, int np) {
     __shared__ int sW[WK_NT / 64];
     __shared__ int sB[WK_NT / 64];
     if (hdr->mode != GRID_MODE_CELLS) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const GridRef g = grid_ref(dir, hdr);
-    const int64_t nb = hdr->nblocks, bchunk = (nb + GRID_PARTS - 1) / GRID_PARTS;
+    const int64_t nb = hdr->nblocks, bchunk = (nb + np - 1) / np;
     const int64_t b0 = blockIdx.x * bchunk, b1 = min(nb, b0 + bchunk);
     int bsum = 0;
     for (int64_t b = b0 + wave; b < b1; b += WK_NT / 64) {
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(WK_NT) void k_walk_count(const int32_t* __restrict_
         if (lane == 0) counts[b] = k;
         bsum += k;
     }
-    const int64_t vchunk = (n + GRID_PARTS - 1) / GRID_PARTS;
+    const int64_t vchunk = (n + np - 1) / np;
     const int64_t v0 = blockIdx.x * vchunk, v1 = min(n, v0 + vchunk);
     int lc = 0;
     for (int64_t i = v0 + tid; i < v1; i += WK_NT) lc += left_out(coords, g, i);
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(WK_NT) void k_walk_count(const int32_t* __restrict_
 // The stores of the walk: the row (order) and packed coordinates (wc) of every voxel -- block
 // voxels from their block's start, column by column, then the left-out voxels after all block
 // voxels. Every workgroup sums the partials before it (and all block partials) itself.
-// Workgroups from GRID_PARTS on carry the neighbour-table probe (pj), when asked for: the walk is
+// Workgroups from np on carry the neighbour-table probe (pj), when asked for: the walk is
 // latency-bound and the probe bound by its table stores, so the two share the launch (2-3 % off
 // the table + plan call, against the probe as a launch of its own; a third of the probe on the
 // count launch instead measured the same).
@@ -100,12 +100,12 @@ __global__ __launch_bounds__(WK_NT) void k_walk_emit(const int32_t* __restrict__
                                                      const int32_t* __restrict__ cell_of,
                                                      const int32_t* __restrict__ parts, int32_t* __restrict__ order,
                                                      uint64_t* __restrict__ wc, int32_t* __restrict__ list_n,
-                                                     ProbeJob pj) {
+                                                     ProbeJob pj, int np) {
     __shared__ int sW[WK_NT / 64];
     __shared__ int sS[3][WK_NT / 64];
     __shared__ int sStart[WK_NT];
-    if (blockIdx.x >= GRID_PARTS) {
-        const int64_t i = pj.v0 + (int64_t)(blockIdx.x - GRID_PARTS) * WK_NT + threadIdx.x;
+    if ((int)blockIdx.x >= np) {
+        const int64_t i = pj.v0 + (int64_t)(blockIdx.x - np) * WK_NT + threadIdx.x;
         if (i < pj.v1) probe_voxel(coords, n, i, dir, hdr, pj.hash, pj.nbr);
         return;
     }
@@ -113,15 +113,13 @@ __global__ __launch_bounds__(WK_NT) void k_walk_emit(const int32_t* __restrict__
     if (hdr->mode != GRID_MODE_CELLS) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const GridRef g = grid_ref(dir, hdr);
-    const int64_t nb = hdr->nblocks, bchunk = (nb + GRID_PARTS - 1) / GRID_PARTS;
+    const int64_t nb = hdr->nblocks, bchunk = (nb + np - 1) / np;
     const int64_t b0 = blockIdx.x * bchunk, b1 = min(nb, b0 + bchunk);
     int base = 0, placed = 0, lbase = 0;
     {
-        constexpr int PPT = GRID_PARTS / WK_NT;
         int bb = 0, ball = 0, lb = 0;
-#pragma unroll
-        for (int k = 0; k < PPT; ++k) {
-            const int p = tid * PPT + k;
+#pragma unroll 4
+        for (int p = tid; p < np; p += WK_NT) {
             const int vb = parts[p], vl = parts[GRID_PARTS + p];
             ball += vb;
             if (p < (int)blockIdx.x) { bb += vb; lb += vl; }
@@ -166,7 +164,7 @@ __global__ __launch_bounds__(WK_NT) void k_walk_emit(const int32_t* __restrict__
         }
         __syncthreads();   // sStart is rewritten by the next round
     }
-    const int64_t vchunk = (n + GRID_PARTS - 1) / GRID_PARTS;
+    const int64_t vchunk = (n + np - 1) / np;
     const int64_t v0 = blockIdx.x * vchunk, v1 = min(n, v0 + vchunk);
     for (int64_t r0 = v0; r0 < v1; r0 += WK_NT) {
         const int64_t i = r0 + tid;
@@ -842,18 +840,19 @@ static int plan_on_grid(const int32_t* nbr, const int32_t* coords, int64_t n, vo
     const PlanView pv = carve_plan(plan, n_tiles);
     // the table probe, when asked for, rides on the walk's emit launch
     ProbeJob pj;
-    int64_t ge = GRID_PARTS;
+    const int np = grid_parts(n);
+    int64_t ge = np;
     if (probe && probe->nbr) {
         pj = *probe;
         pj.v0 = 0;
         pj.v1 = n;
         ge += ceil_div(n, WK_NT);
     }
-    hipLaunchKernelGGL(k_walk_count, dim3(GRID_PARTS), dim3(WK_NT), 0, s, coords, n, dir, gt.hdr, ps.counts,
-                       ps.pres, gt.parts);
+    hipLaunchKernelGGL(k_walk_count, dim3((unsigned)np), dim3(WK_NT), 0, s, coords, n, dir, gt.hdr, ps.counts,
+                       ps.pres, gt.parts, np);
     TSP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_walk_emit, dim3((unsigned)ge), dim3(WK_NT), 0, s, coords, n, dir, gt.hdr, ps.counts,
-                       ps.pres, ps.cell_of, gt.parts, ps.order, ps.wc, list_n, pj);
+                       ps.pres, ps.cell_of, gt.parts, ps.order, ps.wc, list_n, pj, np);
     TSP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_plan_window, dim3((unsigned)n_tiles), dim3(HB_PLAN_NT), 0, s, n, ps.order, ps.wc, dir,
                        ps.pres, gt.hdr, pv, list, list_n);
