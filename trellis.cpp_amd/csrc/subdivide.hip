@@ -15,8 +15,8 @@
 namespace tsp {
 namespace {
 
-constexpr int SD_THREADS = 256;
-constexpr int SD_PER_THREAD = 4;
+constexpr int SD_THREADS = 1024;
+constexpr int SD_PER_THREAD = 1;
 constexpr int SD_ITEMS = SD_THREADS * SD_PER_THREAD;   // parents per block
 
 __device__ __forceinline__ uint32_t octant_bits(const uint8_t* __restrict__ mask, int64_t i) {
@@ -80,36 +80,45 @@ __global__ __launch_bounds__(SD_THREADS) void k_scan_block_sums(int32_t* block_s
     }
 }
 
+// A block's children are listed in LDS (parent of the block and octant, in order), then written a
+// word at a time along the outputs, so that every store of a wave is one piece of memory: 290 K
+// parents, 1.19 M children 12 us; each thread writing its own four parents' children took 20.
 __global__ __launch_bounds__(SD_THREADS) void k_emit_children(
     const uint8_t* __restrict__ mask, const int32_t* __restrict__ coords, int64_t n,
     const int32_t* __restrict__ block_offsets, int32_t* __restrict__ mstart,
     int32_t* __restrict__ child, int32_t* __restrict__ gidx) {
-    const int64_t p0 = (int64_t)blockIdx.x * SD_ITEMS + (int64_t)threadIdx.x * SD_PER_THREAD;
+    __shared__ int32_t sC[3 * SD_ITEMS];          // the block's parents
+    __shared__ uint16_t sList[8 * SD_ITEMS];      // octant + 8 parent of each child
+    const int64_t b0 = (int64_t)blockIdx.x * SD_ITEMS;
+    const int tid = threadIdx.x, items = (int)min<int64_t>(SD_ITEMS, n - b0);
+    for (int k = tid; k < 3 * items; k += SD_THREADS) sC[k] = coords[3 * b0 + k];
+    const int l0 = tid * SD_PER_THREAD;
     uint32_t bits[SD_PER_THREAD];
     int32_t c = 0;
 #pragma unroll
     for (int k = 0; k < SD_PER_THREAD; ++k) {
-        bits[k] = (p0 + k < n) ? octant_bits(mask, p0 + k) : 0u;
+        bits[k] = (l0 + k < items) ? octant_bits(mask, b0 + l0 + k) : 0u;
         c += __popc(bits[k]);
     }
     int32_t tot;
-    int32_t m = block_offsets[blockIdx.x] + block_exclusive_scan(c, &tot);
+    int32_t m = block_exclusive_scan(c, &tot);
+    const int32_t m0 = block_offsets[blockIdx.x];
 #pragma unroll
     for (int k = 0; k < SD_PER_THREAD; ++k) {
-        const int64_t i = p0 + k;
-        if (i >= n) break;
-        mstart[i] = m;
-        const int32_t x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
+        if (l0 + k >= items) break;
+        mstart[b0 + l0 + k] = m0 + m;
         uint32_t b = bits[k];
         while (b) {
-            const int o = __builtin_ctz(b);
+            sList[m++] = (uint16_t)(__builtin_ctz(b) + 8 * (l0 + k));
             b &= b - 1;
-            child[3 * (int64_t)m + 0] = 2 * x + (o & 1);
-            child[3 * (int64_t)m + 1] = 2 * y + ((o >> 1) & 1);
-            child[3 * (int64_t)m + 2] = 2 * z + ((o >> 2) & 1);
-            gidx[m] = (int32_t)(o + 8 * i);
-            ++m;
         }
+    }
+    __syncthreads();
+    for (int k = tid; k < tot; k += SD_THREADS) gidx[(int64_t)m0 + k] = (int32_t)(8 * b0 + sList[k]);
+    for (int d = tid; d < 3 * tot; d += SD_THREADS) {
+        const int k = d / 3, a = d - 3 * k;
+        const int e = sList[k];
+        child[3 * (int64_t)m0 + d] = 2 * sC[3 * (e >> 3) + a] + ((e >> a) & 1);
     }
 }
 
