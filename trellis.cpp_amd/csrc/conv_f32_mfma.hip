@@ -43,9 +43,13 @@ __global__ __launch_bounds__(64 * KG) void k_conv_f32_mfma(const float* __restri
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int r32 = lane & 31, h = lane >> 5;
-    const int64_t tile = blockIdx.x / n_ctiles;
-    const int c0 = (int)(blockIdx.x % n_ctiles) * 32 * CB;
+    // Workgroup ids go round-robin over the 8 XCDs: each XCD takes a contiguous range of units, whose
+    // neighbour rows its L2 then holds (the grid is a multiple of 8).
+    const int64_t unit = (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    const int64_t tile = unit / n_ctiles;
+    const int c0 = (int)(unit % n_ctiles) * 32 * CB;
     const int64_t row0 = tile * 32 * RB;
+    if (row0 >= n) return;
     const uint32_t un = (uint32_t)n;
 
     // whether the padding row holds a NaN (an exact zero row, pad.zero, never does)
@@ -211,10 +215,10 @@ int launch_cb(const float* feats, int64_t n, int ci, const int32_t* nbr, const f
     const int64_t waves_wanted = 16LL * cu_count_f32();
     const int64_t t64 = ceil_div(n, 64) * n_ctiles, t32 = ceil_div(n, 32) * n_ctiles;
     if (t64 >= waves_wanted)
-        hipLaunchKernelGGL((k_conv_f32_mfma<ODT, 2, CB, 1>), dim3((unsigned)t64), dim3(64), 0, s, feats, n, ci,
+        hipLaunchKernelGGL((k_conv_f32_mfma<ODT, 2, CB, 1>), dim3((unsigned)(ceil_div(t64, 8) * 8)), dim3(64), 0, s, feats, n, ci,
                            nbr, weight, bias, co, out, n_ctiles, pad);
     else
-        hipLaunchKernelGGL((k_conv_f32_mfma<ODT, 1, CB, 4>), dim3((unsigned)t32), dim3(256), 0, s, feats, n, ci,
+        hipLaunchKernelGGL((k_conv_f32_mfma<ODT, 1, CB, 4>), dim3((unsigned)(ceil_div(t32, 8) * 8)), dim3(256), 0, s, feats, n, ci,
                            nbr, weight, bias, co, out, n_ctiles, pad);
     TSP_CHECK_LAUNCH();
     return TSP_OK;
@@ -238,7 +242,7 @@ int f32_mfma_launch(int fdt, int wdt, int odt, const void* feats, int64_t n, int
                     const void* weight, const float* bias, int co, void* out, hipStream_t s, PadRow pad) {
     if (!nbr || !f32_mfma_fits(fdt, wdt, ci, co, feats, weight)) return TSP_ERR_UNSUPPORTED;
     // grid.x is a tile count below 2^31: n < 2^31 rows, 32-row tiles, co / 32 column tiles
-    if (ceil_div(n, 32) * (co / 32) >= ((int64_t)1 << 31)) return TSP_ERR_UNSUPPORTED;
+    if (ceil_div(n, 32) * (co / 32) >= ((int64_t)1 << 31) - 8) return TSP_ERR_UNSUPPORTED;
     const float* f = static_cast<const float*>(feats);
     const float* w = static_cast<const float*>(weight);
     switch (odt) {
