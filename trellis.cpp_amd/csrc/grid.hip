@@ -175,7 +175,12 @@ __global__ __launch_bounds__(GB_NT) void k_grid_apply(GridHdr* __restrict__ hdr,
                                                       int32_t* __restrict__ cell_of, int64_t block_cap, int np) {
     __shared__ int sW[2][GB_NT / 64];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    bool cells = hdr->mode == GRID_MODE_CELLS;
+    // Read once a workgroup: workgroup 0 may write the fallback while another one starts, which then
+    // takes it as a whole (the same answer it would find) and never by some of its waves alone.
+    __shared__ int sMode;
+    if (tid == 0) sMode = hdr->mode;
+    __syncthreads();
+    bool cells = sMode == GRID_MODE_CELLS;
     int64_t nblocks = 0;
     int run = 0;
     if (cells) {
