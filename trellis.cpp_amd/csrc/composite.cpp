@@ -231,7 +231,7 @@ int c2s_walk(const float* x, int64_t n, int cin, const int32_t* nbr, const void*
     OctantPlan op;
     void* oplan = nullptr;
     int32_t *members = nullptr, *ocounts = nullptr, *oct_tiles = nullptr;
-    const bool oct_plan = octants && octant_plan_spec(n, m, cin, cout, op);
+    bool oct_plan = octants && octant_plan_spec(n, m, cin, cout, op);
     if (oct_plan) {
         oplan = ws.take(op.plan_bytes);
         members = static_cast<int32_t*>(ws.take(op.member_bytes));
@@ -239,6 +239,7 @@ int c2s_walk(const float* x, int64_t n, int cin, const int32_t* nbr, const void*
         oct_tiles = static_cast<int32_t*>(ws.take(4));
     }
     if (!ws.base) return TSP_OK;
+    if (reinterpret_cast<uintptr_t>(ws.base) & 15) oct_plan = false;   // (a plan is 16-byte aligned)
     int st;
     const void* p2 = pk2 ? pk2 : w.conv2_packed;
     if (part & TSP_C2S_PART_FRONT) {
@@ -249,8 +250,8 @@ int c2s_walk(const float* x, int64_t n, int cin, const int32_t* nbr, const void*
             p1 = pk1;
         }
         auto al = [](const void* q, uintptr_t a) { return (reinterpret_cast<uintptr_t>(q) & (a - 1)) == 0; };
-        TSP_REQUIRE(!oct_plan || (al(p1, 16) && al(mask, 8) && al(h0, 16)), TSP_ERR_INVALID,
-                    "tsp_c2s: packed conv1 weights and the workspace must be 16-byte aligned, the mask 8-byte");
+        TSP_REQUIRE(!oct_plan || (al(p1, 16) && al(mask, 8)), TSP_ERR_INVALID,
+                    "tsp_c2s: packed conv1 weights must be 16-byte aligned, the mask 8-byte");
         if (oct_plan) st = octant_plan_build(op, plan, n, nbr, mask, oplan, members, ocounts, oct_tiles, s);
         else if (octants) st = octant_blocks(plan, n, mask, blocks, s);
         if (st) return st;
