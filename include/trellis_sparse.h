@@ -390,7 +390,10 @@ typedef struct {
     const void* conv2_packed;
 } tsp_c2s_weights;
 
-/* Workspace tsp_c2s needs (only the dtypes and *_packed of w are read). */
+/* Workspace tsp_c2s uses (only the dtypes and *_packed of w are read), for the very n and m of the
+ * call: with d_plan, 16-bit conv1 weights and cout % 128 == 0 it may hold a plan of conv1's kept
+ * (parent, octant) rows, which depends on m / n. A workspace that is short of that part alone (one
+ * sized for more children, say) is accepted: conv1 then runs without it, to the same bits. */
 size_t tsp_c2s_workspace_bytes(int64_t n, int64_t m, int cin, int cout, const tsp_c2s_weights* w,
                                int has_plan, int has_child_plan, int flags);
 /* The features of SparseResBlockC2S3d (replaces the feature half of trellis::sparse_c2s,

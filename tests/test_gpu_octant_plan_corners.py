@@ -1,0 +1,96 @@
+"""The C2S block's octant plan (csrc/plan.hip) where it is not the usual call: a workspace without
+room for it."""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _al(b):
+    return (b + 255) // 256 * 256
+
+
+def _without_plan(n, m, cin, cout):
+    """The C2S workspace without the octant plan (both plans given, packed 16-bit weights): norm1's
+    output, conv1's rows in f32 where its stores do not normalise, conv2's input, the block words."""
+    return (_al(2 * n * cin) + (0 if cout in (64, 128) else _al(4 * m * cout)) + _al(2 * m * cout)
+            + _al(16 * -(-n // 512)))
+
+
+def _block(tsp, shells, n, cin, cout, keep, key="bf16", seed=0):
+    """A C2S block with device tensors: n parents of a shell, octant o kept with probability keep[o]."""
+    import torch
+    dt = torch.bfloat16 if key == "bf16" else torch.float16
+    rng = np.random.default_rng(n + cin + seed)
+    coords = shells.sphere_shell(96, 48.0, 34.0, 36.4 if n > 12000 else 35.6)
+    assert len(coords) >= n
+    c = torch.from_numpy(np.ascontiguousarray(coords[:n], np.int32)).cuda()
+    mask = torch.from_numpy((rng.random((n, 8)) < np.asarray(keep)).astype(np.uint8).reshape(-1)).cuda()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + seed)
+    rand = lambda shape, std, d: (torch.randn(shape, generator=g, device="cuda") * std).to(d)
+    p = {"norm1.weight": 1 + rand((cin,), 0.1, torch.float32), "norm1.bias": rand((cin,), 0.1, torch.float32),
+         "conv1.weight": rand((8 * cout, 27, cin), (27 * cin) ** -0.5, dt), "conv1.bias": rand((8 * cout,), 0.1, torch.float32),
+         "conv2.weight": rand((cout, 27, cout), (27 * cout) ** -0.5, dt), "conv2.bias": rand((cout,), 0.1, torch.float32)}
+    p["conv1.packed"], p["conv2.packed"] = tsp.conv_weight_pack(p["conv1.weight"]), tsp.conv_weight_pack(p["conv2.weight"])
+    nbr, plan = tsp.rulebook_build_planned(c)
+    child, gidx, mstart = tsp.subdivide(mask, c)
+    cnbr, cplan = tsp.rulebook_build_planned(child)
+    x = rand((n, cin), 1.0, torch.float32)
+    return {"n": n, "m": len(gidx), "cin": cin, "cout": cout, "x": x, "nbr": nbr, "plan": plan, "mask": mask,
+            "gidx": gidx, "mstart": mstart, "cnbr": cnbr, "cplan": cplan, "p": p}
+
+
+def _weights(tsp, p):
+    from trellis_cpp_amd import C2SWeights
+    ptr, code = (lambda t: ctypes.c_void_p(t.data_ptr())), tsp.dtype_code
+    return C2SWeights(ptr(p["norm1.weight"]), ptr(p["norm1.bias"]), ptr(p["conv1.weight"]), code(p["conv1.weight"].dtype),
+                      ptr(p["conv1.bias"]), ptr(p["conv1.packed"]), ptr(p["conv2.weight"]), code(p["conv2.weight"].dtype),
+                      ptr(p["conv2.bias"]), ptr(p["conv2.packed"]))
+
+
+def _run(tsp, b, ws, ws_bytes):
+    """tsp_c2s on the workspace's first ws_bytes -> (status, out)."""
+    import torch
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    out = torch.full((b["m"], b["cout"]), float("nan"), device="cuda")
+    st = tsp.lib().tsp_c2s(ptr(b["x"]), b["n"], b["cin"], ptr(b["nbr"]), ptr(b["plan"]), ptr(b["mask"]), ptr(b["mstart"]),
+                           ptr(b["gidx"]), b["m"], b["cout"], ptr(b["cnbr"]), ptr(b["cplan"]),
+                           ctypes.byref(_weights(tsp, b["p"])), ptr(out), ptr(ws), ws_bytes, 0,
+                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return st, out
+
+
+def _bytes(tsp, b, m=None):
+    return tsp.lib().tsp_c2s_workspace_bytes(b["n"], b["m"] if m is None else m, b["cin"], b["cout"],
+                                             ctypes.byref(_weights(tsp, b["p"])), 1, 1, 0)
+
+
+@pytest.mark.parametrize("n,cin,cout", [(14001, 256, 128), (8001, 512, 256)])
+def test_workspace_without_the_plan(gpu_lib, shells, n, cin, cout):
+    """A workspace of the size without the octant plan -- what callers asked for before there was one,
+    or sized for more children than there are -- is accepted, gives the same bits and is not written
+    past its end; a byte less is refused."""
+    import torch
+    print(f"[octant plan] small workspace n={n} {cin}->{cout}", flush=True)
+    b = _block(gpu_lib, shells, n, cin, cout, [0.5] * 8)
+    full, less = _bytes(gpu_lib, b), _without_plan(n, b["m"], cin, cout)
+    assert less < full, "the case is meant to take an octant plan"
+    ws = torch.full((full,), 0xA5, dtype=torch.uint8, device="cuda")
+    st, want = _run(gpu_lib, b, ws, full)
+    assert st == 0
+    ws.fill_(0xA5)
+    for size in (less, full - 1):
+        st, got = _run(gpu_lib, b, ws, size)
+        assert st == 0 and torch.equal(got, want)
+    assert bool((ws[less:] == 0xA5).all())
+    assert _run(gpu_lib, b, ws, less - 1)[0] == 5
+    # sized for every octant kept, where conv1 takes no plan
+    assert _bytes(gpu_lib, b, 8 * n) == _without_plan(n, 8 * n, cin, cout)
+    st, got = _run(gpu_lib, b, ws, min(full, _bytes(gpu_lib, b, 8 * n)))
+    assert st == 0 and torch.equal(got, want)

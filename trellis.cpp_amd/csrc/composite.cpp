@@ -7,6 +7,7 @@
 // conv weights under TSP_BLOCK_CAST_F32 (the reference's g_sparse_cast_f32 casts them, w32,
 // sparse.cpp:16-19).
 #include <algorithm>
+#include <cstdint>
 
 #include "blocks_internal.hpp"
 #include "common.hpp"
@@ -16,10 +17,12 @@ namespace tsp {
 namespace {
 
 // Workspace carving: a null base only sizes (take() returns null), a real one hands out pieces.
+// limit: the bytes there are; pieces that a block can do without are taken only where they fit.
 struct Carve {
     char* base;
+    size_t limit;
     size_t off = 0;
-    explicit Carve(void* b) : base(static_cast<char*>(b)) {}
+    explicit Carve(void* b, size_t bytes = SIZE_MAX) : base(static_cast<char*>(b)), limit(bytes) {}
     void* take(size_t bytes) {
         void* p = base ? base + off : nullptr;
         off += (bytes + 255) / 256 * 256;
@@ -232,11 +235,17 @@ int c2s_walk(const float* x, int64_t n, int cin, const int32_t* nbr, const void*
     void* oplan = nullptr;
     int32_t *members = nullptr, *ocounts = nullptr, *oct_tiles = nullptr;
     bool oct_plan = octants && octant_plan_spec(n, m, cin, cout, op);
+    const size_t before_plan = ws.off;
     if (oct_plan) {
         oplan = ws.take(op.plan_bytes);
         members = static_cast<int32_t*>(ws.take(op.member_bytes));
         ocounts = static_cast<int32_t*>(ws.take(op.count_bytes));
         oct_tiles = static_cast<int32_t*>(ws.take(4));
+        // (the last pieces: a workspace without room for them runs conv1 on the parents' plan)
+        if (ws.off > ws.limit) {
+            ws.off = before_plan;
+            oct_plan = false;
+        }
     }
     if (!ws.base) return TSP_OK;
     if (reinterpret_cast<uintptr_t>(ws.base) & 15) oct_plan = false;   // (a plan is 16-byte aligned)
@@ -375,13 +384,19 @@ extern "C" int tsp_convnext(const void* d_x, int x_dtype, int64_t n, int c, cons
                            workspace_bytes, flags, stream);
 }
 
+// limit 0: without the pieces that tsp_c2s can do without
+static size_t c2s_bytes(int64_t n, int64_t m, int cin, int cout, const tsp_c2s_weights& w, bool has_plan,
+                        bool has_child_plan, int flags, size_t limit) {
+    Carve ws(nullptr, limit);
+    c2s_walk(nullptr, n, cin, nullptr, plan_flag(has_plan), nullptr, nullptr, nullptr, m, cout, nullptr,
+             plan_flag(has_child_plan), w, nullptr, nullptr, TSP_BF16, flags, ws, nullptr);
+    return ws.off;
+}
+
 extern "C" size_t tsp_c2s_workspace_bytes(int64_t n, int64_t m, int cin, int cout, const tsp_c2s_weights* w,
                                           int has_plan, int has_child_plan, int flags) {
     if (n <= 0 || m < 0 || cin <= 0 || cout <= 0 || !w) return 0;
-    Carve ws(nullptr);
-    c2s_walk(nullptr, n, cin, nullptr, plan_flag(has_plan), nullptr, nullptr, nullptr, m, cout, nullptr,
-             plan_flag(has_child_plan), *w, nullptr, nullptr, TSP_BF16, flags, ws, nullptr);
-    return ws.off;
+    return c2s_bytes(n, m, cin, cout, *w, has_plan, has_child_plan, flags, SIZE_MAX);
 }
 
 extern "C" int tsp_c2s_part(const float* d_x, int64_t n, int cin, const int32_t* d_nbr, const void* d_plan,
@@ -415,10 +430,10 @@ extern "C" int tsp_c2s_part(const float* d_x, int64_t n, int cin, const int32_t*
                 TSP_ERR_INVALID, "tsp_c2s: the rounded copy of out aliases another buffer");
     TSP_REQUIRE((reinterpret_cast<uintptr_t>(d_out16) & 15) == 0, TSP_ERR_INVALID,
                 "tsp_c2s: the rounded copy of out must be 16-byte aligned");
-    const size_t need = tsp_c2s_workspace_bytes(n, m, cin, cout, w, d_plan != nullptr, d_child_plan != nullptr, flags);
+    const size_t need = c2s_bytes(n, m, cin, cout, *w, d_plan != nullptr, d_child_plan != nullptr, flags, 0);
     TSP_REQUIRE(d_workspace && workspace_bytes >= need, TSP_ERR_WORKSPACE, "tsp_c2s: workspace %zu < %zu bytes",
                 workspace_bytes, need);
-    Carve ws(d_workspace);
+    Carve ws(d_workspace, workspace_bytes);
     return c2s_walk(d_x, n, cin, d_nbr, d_plan, d_mask, d_mstart, d_gidx, m, cout, d_child_nbr, d_child_plan, *w,
                     d_out, d_out16, out16_dtype, flags, ws, as_stream(stream), part, TileRange{t0, nt});
 }
