@@ -1,5 +1,5 @@
 """The C2S block's octant plan (csrc/plan.hip) where it is not the usual call: a workspace without
-room for it."""
+room for it; masks that keep some octants far more often than others."""
 from __future__ import annotations
 
 import ctypes
@@ -94,3 +94,59 @@ def test_workspace_without_the_plan(gpu_lib, shells, n, cin, cout):
     assert _bytes(gpu_lib, b, 8 * n) == _without_plan(n, 8 * n, cin, cout)
     st, got = _run(gpu_lib, b, ws, min(full, _bytes(gpu_lib, b, 8 * n)))
     assert st == 0 and torch.equal(got, want)
+
+
+# keep probabilities of the octants, and whether the plan then pays: only where its fullest octant has
+# clearly fewer tiles than the parents (large grid) or all octants together do (small grid)
+MASKS = {"half": [0.5] * 8, "rare": [0.3] * 8, "two rates": [0.4, 0.6] * 4, "one full": [1.0] + [0.05] * 7,
+         "half full": [0.9] * 4 + [0.1] * 4, "none": [0.0, 0.001] + [0.5] * 6}
+
+
+def _front_us(tsp, b, ws, ws_bytes):
+    """The shortest of five runs of the block's front part (conv1 and its norms), us."""
+    import torch
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    out = torch.empty((b["m"], b["cout"]), device="cuda")
+    best = float("inf")
+    for _ in range(5):
+        t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        t0.record()
+        st = tsp.lib().tsp_c2s_part(ptr(b["x"]), b["n"], b["cin"], ptr(b["nbr"]), ptr(b["plan"]), ptr(b["mask"]),
+                                    ptr(b["mstart"]), ptr(b["gidx"]), b["m"], b["cout"], ptr(b["cnbr"]), ptr(b["cplan"]),
+                                    ctypes.byref(_weights(tsp, b["p"])), ptr(out), None, 2, ptr(ws), ws_bytes, 0, 1, 0, -1,
+                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        t1.record()
+        torch.cuda.synchronize()
+        assert st == 0
+        best = min(best, t0.elapsed_time(t1) * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("n,cin,cout", [(24001, 256, 128), (12001, 512, 256), (9001, 256, 384)])
+@pytest.mark.parametrize("keep", list(MASKS))
+def test_uneven_octants(gpu_lib, shells, n, cin, cout, keep):
+    """Each octant's tiles are its own (none is empty or reads its rows from memory), a plan that does
+    not pay is not run, and the block is the same bits either way. A mask that keeps the octants
+    unevenly runs about as fast as with a workspace without room for the plan: within a factor of 2
+    here, where tiles of parents far apart, or eight times the fullest octant's tiles, take 3 to 6."""
+    import torch
+    print(f"[octant plan] {keep} n={n} {cin}->{cout}", flush=True)
+    b = _block(gpu_lib, shells, n, cin, cout, MASKS[keep])
+    full, less = _bytes(gpu_lib, b), _without_plan(n, b["m"], cin, cout)
+    ws = torch.empty(full, dtype=torch.uint8, device="cuda")
+    st, got = _run(gpu_lib, b, ws, full)
+    assert st == 0
+    if full > less:   # (the plan's state is the first of its pieces)
+        state = ws[less:less + 37 * 4].view(torch.int32).tolist()
+        fits, spare, direct, total, most = state[:5]
+        tiles, base, rows, count = (np.array(state[5 + 8 * k:13 + 8 * k]) for k in range(4))
+        kept = (b["mask"].reshape(n, 8) != 0).sum(0).cpu().numpy()
+        assert np.array_equal(count, kept) and np.array_equal(tiles, -(-kept // rows))
+        assert total == tiles.sum() and most == tiles.max() and np.array_equal(base, np.cumsum(tiles) - tiles)
+        assert direct == 0 and (rows <= 512).all()
+        if fits:
+            assert most <= -(-n // 512)
+        assert bool(fits) == (keep in ("half", "rare", "two rates", "none")) or cout == 384
+    st, want = _run(gpu_lib, b, ws, less)
+    assert st == 0 and torch.equal(got, want)
+    assert _front_us(gpu_lib, b, ws, full) < 2 * _front_us(gpu_lib, b, ws, less) + 50

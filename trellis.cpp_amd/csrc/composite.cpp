@@ -230,17 +230,19 @@ int c2s_walk(const float* x, int64_t n, int cin, const int32_t* nbr, const void*
     // with octant stores: which of conv1's row blocks hold a parent keeping each octant (the
     // others' MFMAs for that octant's channels are skipped; their outputs are never stored)
     auto* blocks = octants ? static_cast<uint32_t*>(ws.take((size_t)ceil_div(n, HB_M) * 4 * 4)) : nullptr;
-    // large blocks instead run conv1 on an octant plan: only the kept (parent, octant) rows
+    // large blocks run conv1 on an octant plan, only the kept (parent, octant) rows, where the mask
+    // leaves enough out
     OctantPlan op;
+    OctantTiles* oct = nullptr;
     void* oplan = nullptr;
-    int32_t *members = nullptr, *ocounts = nullptr, *oct_tiles = nullptr;
+    int32_t *members = nullptr, *ocounts = nullptr;
     bool oct_plan = octants && octant_plan_spec(n, m, cin, cout, op);
     const size_t before_plan = ws.off;
     if (oct_plan) {
+        oct = static_cast<OctantTiles*>(ws.take(sizeof(OctantTiles)));
         oplan = ws.take(op.plan_bytes);
         members = static_cast<int32_t*>(ws.take(op.member_bytes));
         ocounts = static_cast<int32_t*>(ws.take(op.count_bytes));
-        oct_tiles = static_cast<int32_t*>(ws.take(4));
         // (the last pieces: a workspace without room for them runs conv1 on the parents' plan)
         if (ws.off > ws.limit) {
             ws.off = before_plan;
@@ -259,39 +261,27 @@ int c2s_walk(const float* x, int64_t n, int cin, const int32_t* nbr, const void*
             p1 = pk1;
         }
         auto al = [](const void* q, uintptr_t a) { return (reinterpret_cast<uintptr_t>(q) & (a - 1)) == 0; };
-        TSP_REQUIRE(!oct_plan || (al(p1, 16) && al(mask, 8)), TSP_ERR_INVALID,
+        TSP_REQUIRE(!octants || (al(p1, 16) && al(mask, 8)), TSP_ERR_INVALID,
                     "tsp_c2s: packed conv1 weights must be 16-byte aligned, the mask 8-byte");
-        if (oct_plan) st = octant_plan_build(op, plan, n, nbr, mask, oplan, members, ocounts, oct_tiles, s);
+        if (oct_plan) st = octant_plan_build(op, plan, n, nbr, mask, oplan, members, ocounts, blocks, oct, s);
         else if (octants) st = octant_blocks(plan, n, mask, blocks, s);
         if (st) return st;
-        if (norm_in_stores) {
-            TSP_REQUIRE((reinterpret_cast<uintptr_t>(p1) & 15) == 0 &&
-                            (reinterpret_cast<uintptr_t>(mask) & 7) == 0,
-                        TSP_ERR_INVALID, "tsp_c2s: packed conv1 weights must be 16-byte aligned, the mask 8-byte");
+        if (octants) {
             OctantScatter osc;
             osc.mask = mask;
             osc.mstart = mstart;
             osc.cout = cout;
-            osc.norm_silu = true;
+            osc.norm_silu = norm_in_stores;
             osc.norm_eps = 1e-6f;
+            osc.blocks = blocks;
             if (oct_plan) {
-                osc.oct_tiles = oct_tiles;
+                osc.oct = oct;
+                osc.oct_plan = oplan;
                 osc.oct_cap = op.cap;
-            } else {
-                osc.blocks = blocks;
             }
-            st = halo_conv_launch(in1, in2, h0, n, cin, nbr, oct_plan ? oplan : plan, p1, w.conv1_bias, 8 * cout, h2, s,
-                                  osc);
-        } else if (oct_plan) {
-            OctantScatter osc;
-            osc.mask = mask;
-            osc.mstart = mstart;
-            osc.cout = cout;
-            osc.oct_tiles = oct_tiles;
-            osc.oct_cap = op.cap;
-            st = halo_conv_launch(in1, TSP_F32, h0, n, cin, nbr, oplan, p1, w.conv1_bias, 8 * cout, g, s, osc);
-        } else if (octants) {
-            st = planned_octants(h0, in1, n, cin, nbr, plan, p1, w.conv1_bias, cout, mask, mstart, g, blocks, s);
+            st = norm_in_stores
+                     ? halo_conv_launch(in1, in2, h0, n, cin, nbr, plan, p1, w.conv1_bias, 8 * cout, h2, s, osc)
+                     : planned_octants(h0, in1, n, cin, nbr, plan, p1, w.conv1_bias, osc, g, s);
         } else {
             if (cp1.planned)
                 st = tsp_subm_conv3x3_planned_ex(h0, in1, n, cin, nbr, plan, p1, w.conv1_bias, 8 * cout, h1,

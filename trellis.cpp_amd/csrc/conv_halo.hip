@@ -31,46 +31,7 @@ __global__ void k_pack_trailer_clear(uint32_t* __restrict__ trailer) {
     trailer[threadIdx.x] = 0u;
 }
 
-// One workgroup per tile, one thread per position: the octants each position's parent keeps
-// (mask bytes != 0), ORed over each 32-position block (a wave's ballot covers two) into the word
-// of its row group: bit 4 o + b for block b (0..3) of the 128 positions of row group p / 128.
-__global__ __launch_bounds__(HB_M) void k_octant_blocks(const int32_t* __restrict__ vox, int64_t n,
-                                                       const uint8_t* __restrict__ mask,
-                                                       uint32_t* __restrict__ out) {
-    __shared__ uint32_t sw[HB_M / 128];
-    const int64_t tile = blockIdx.x;
-    const int p = threadIdx.x, lane = p & 63, wave = p >> 6;
-    if (p < HB_M / 128) sw[p] = 0u;
-    __syncthreads();
-    const int32_t v = vox[tile * HB_M + p];
-    uint32_t kept = 0;
-    if (v >= 0 && v < n) {
-#pragma unroll
-        for (int o = 0; o < 8; ++o) kept |= (mask[8 * (int64_t)v + o] != 0 ? 1u : 0u) << o;
-    }
-    uint32_t bits = 0;
-    const int b0 = (wave & 1) * 2;   // this wave's first block within its row group
-#pragma unroll
-    for (int o = 0; o < 8; ++o) {
-        const uint64_t b = __ballot((kept >> o) & 1u);
-        bits |= ((uint32_t)(b & 0xffffffffull) != 0u ? 1u : 0u) << (4 * o + b0);
-        bits |= ((uint32_t)(b >> 32) != 0u ? 1u : 0u) << (4 * o + b0 + 1);
-    }
-    if (lane == 0 && bits) atomicOr(&sw[wave >> 1], bits);
-    __syncthreads();
-    if (p < HB_M / 128) out[tile * (HB_M / 128) + p] = sw[p];
-}
-
 }  // namespace
-
-int octant_blocks(const void* plan, int64_t n, const uint8_t* mask, uint32_t* out, hipStream_t s) {
-    const int64_t n_tiles = ceil_div(n, HB_M);
-    if (n_tiles == 0) return TSP_OK;
-    const PlanView pv = carve_plan(const_cast<void*>(plan), n_tiles);
-    hipLaunchKernelGGL(k_octant_blocks, dim3((unsigned)n_tiles), dim3(HB_M), 0, s, pv.vox, n, mask, out);
-    TSP_CHECK_LAUNCH();
-    return TSP_OK;
-}
 
 bool halo_fits(int64_t n, int ci) { return n * (int64_t)ci * 2 < ((int64_t)1 << 32); }
 
@@ -103,6 +64,8 @@ int64_t column_split_tiles(int64_t n_tiles, int nct, int cus) {
     const int64_t fit64 = std::max<int64_t>(1, cus / 8 / (2 * nct)) * (2 * nct);
     return ceil_div(left * 2 * nct, 8) <= fit64 ? t_split : 0;
 }
+
+int conv_cus() { return cu_count(); }
 
 int conv_split_pick(int64_t n, int ci, int co, int ncg) {
     if (n <= 0 || co % (64 * ncg) != 0) return 0;
@@ -156,7 +119,7 @@ int halo_conv_launch(int fdt, int odt, const void* feats, int64_t n, int ci, con
                   "(co=%d cout=%d)", bn128 ? 64 : 32, co, osc.cout);
         return TSP_ERR_UNSUPPORTED;
     }
-    if (osc.oct_tiles && (osc.cout % 128 != 0 || osc.blocks || !all_tiles)) {
+    if (osc.oct && (osc.cout % 128 != 0 || !osc.oct_plan || osc.side != OctantScatter::EITHER || !all_tiles)) {
         set_error("MFMA conv: an octant plan needs cout %% 128 == 0 (cout=%d) and is run whole", osc.cout);
         return TSP_ERR_UNSUPPORTED;
     }
@@ -188,9 +151,16 @@ int halo_conv_launch(int fdt, int odt, const void* feats, int64_t n, int ci, con
     // With a plan, whole rounds of 128-channel units and the tiles left over as 64-channel units
     // (kernels where either width runs: not the row norms, which need whole rows in a workgroup)
     if (!all_tiles) return fn(odt, planned, feats, n, ci, nbr, plan, weight, bias, co, out, s, osc, skip, pad, ln, tr);
-    if (planned && bn128 && !ln.w && !osc.norm_silu && !osc.oct_tiles) {
+    if (planned && bn128 && !ln.w && !osc.norm_silu) {
         const int64_t t_split = column_split_tiles(ceil_div(n, HB_M), co / 128, cu_count());
         if (t_split > 0) {
+            if (osc.oct) {   // an octant plan takes no column split
+                osc.side = OctantScatter::OCTANTS;
+                if (int st = fn(odt, planned, feats, n, ci, nbr, plan, weight, bias, co, out, s, osc, skip, pad, ln,
+                                TileRange{}))
+                    return st;
+                osc.side = OctantScatter::PARENTS;
+            }
             if (int st = fn(odt, planned, feats, n, ci, nbr, plan, weight, bias, co, out, s, osc, skip, pad, ln,
                             TileRange{0, t_split}))
                 return st;

@@ -110,13 +110,20 @@ __device__ __forceinline__ void conv_grid(
     // workgroup per CU, otherwise one workgroup per pair.
     int64_t total = n_tiles * n_ctiles;
     if constexpr (EPI == 1 || EPI == 5) {
-        if (osc.oct_tiles) {   // an octant plan: its tile count is known on the device only
-            total = min<int64_t>(n_tiles, *osc.oct_tiles) * n_ctiles;
+        if (!octant_side(osc, plan)) return;
+        if (osc.oct) {   // (never more units than on the parents' plan)
+            total = (int64_t)osc.oct->most * n_ctiles;
             per_xcd = (total + 7) / 8;
         }
     }
     const int xcd = (int)(blockIdx.x % 8);
-    const int64_t xlo = xcd * per_xcd, xhi = xlo + per_xcd < total ? xlo + per_xcd : total;
+    const int64_t xlo = xcd * per_xcd;
+    int64_t xhi = xlo + per_xcd < total ? xlo + per_xcd : total;
+    if constexpr (EPI == 1 || EPI == 5) {
+        // unit lin is tile lin / n_ctiles of its column's octant, which ends with the octant's tiles
+        if (osc.oct)
+            xhi = min(xhi, (int64_t)osc.oct->tiles[(int)((xlo + blockIdx.x / 8) % n_ctiles) * BN / osc.cout] * n_ctiles);
+    }
     conv_tiles<BF16, BN, ODT, PLANNED, RB, CB, PD, SP, STG, EPI>(
         feats, n, ci, nbr, plan, weight, bias, co, out, n_ctiles, xlo + blockIdx.x / 8,
         gridDim.x / 8, xhi, sH0, sH1, sL, sRed, osc, skip, pad, ln);
@@ -227,14 +234,12 @@ __device__ __forceinline__ void conv_tiles(
     // with an octant scatter, the wave's channels lie in octant oct, from column ocol of a child
     const int oct = EPI == 1 || EPI == 4 || EPI == 5 ? c0 / osc.cout : 0;
     const int ocol = EPI == 1 || EPI == 4 || EPI == 5 ? c0 - oct * osc.cout : 0;
-    // the plan's tile of unit lin: on an octant plan, tile k of the unit's octant is 8 k + octant
-    const int unit_oct = (EPI == 1 || EPI == 5) && osc.oct_tiles ? (int)(lin0 % n_ctiles) * BN / osc.cout : -1;
-    auto plan_tile = [&](int64_t lin) -> int64_t {
-        if constexpr (EPI == 1 || EPI == 5) {
-            if (unit_oct >= 0) return lin / n_ctiles * 8 + unit_oct;
-        }
-        return lin / n_ctiles;
-    };
+    // the plan's tile of unit lin: on an octant plan, counted from the first of the column's octant
+    int tile0 = 0;
+    if constexpr (EPI == 1 || EPI == 5) {
+        if (osc.oct) tile0 = osc.oct->base[(int)(lin0 % n_ctiles) * BN / osc.cout];
+    }
+    auto plan_tile = [&](int64_t lin) -> int64_t { return tile0 + lin / n_ctiles; };
     const int nkc = ci / HB_KC;
     // The reference's absent taps read the padding row 0 * feats[0] (submconv_pad,
     // sparse.cpp:81-85), zeros here. Where row 0 holds an Inf or a NaN that row is NaN in those
@@ -1026,7 +1031,7 @@ template <bool BF16, int BN, int ODT, bool PLANNED>
 int launch(const void* feats, int64_t n, int ci, const int32_t* nbr, const void* plan,
            const void* weight, const float* bias, int co, void* out, hipStream_t s, OctantScatter osc,
            SkipAdd skip, PadRow pad, RowNorm ln, TileRange tr) {
-    const int64_t all_tiles = osc.oct_tiles ? osc.oct_cap : ceil_div(n, HB_M);   // (an octant plan: of each octant)
+    const int64_t all_tiles = ceil_div(n, HB_M);
     // a stored plan's tiles [t0, t0 + n_tiles): its per-tile arrays (and the octant block words)
     // start at tile t0, and the kernel's tile indices count from there
     const int64_t t0 = PLANNED ? tr.t0 : 0;
@@ -1042,7 +1047,7 @@ int launch(const void* feats, int64_t n, int ci, const int32_t* nbr, const void*
     const int64_t per_xcd = ceil_div(total, 8);
     PlanView pv{};
     if (plan) {
-        pv = carve_plan(const_cast<void*>(plan), osc.oct_tiles ? 8 * all_tiles : all_tiles);
+        pv = carve_plan(const_cast<void*>(plan), all_tiles);
         pv.hdr += t0 * 4;
         pv.rowof += t0 * HB_SLOTS;
         pv.slots += t0 * HB_SLOT_TABLE;

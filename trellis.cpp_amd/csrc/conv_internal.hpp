@@ -78,6 +78,17 @@ constexpr int HB_PACK_TRAILER = 256;
 inline size_t packed_weight_bytes(int ci, int co) { return (size_t)kTaps * ci * co * 2 + HB_PACK_TRAILER; }
 // Packs [co][27][ci] 16-bit weights of dtype wdt (ci % 16 == 0, co % 32 == 0) and writes the trailer.
 int halo_weight_pack(const void* w, int wdt, int ci, int co, void* packed, hipStream_t s);
+// The state of an octant plan, on the device.
+struct OctantTiles {
+    int32_t fits;         // the plan's tiles fit their space and are few enough to pay
+    int32_t spare;        // how many of them may read their rows from memory (rows past HB_SLOTS)
+    int32_t direct;       // how many do
+    int32_t total, most;  // tiles of all octants; of the octant that has most
+    int32_t tiles[8];     // of each octant
+    int32_t base[8];      // its first tile
+    int32_t rows[8];      // parents of one of its tiles (up to HB_M)
+    int32_t count[8];     // parents that keep it
+};
 // Output rows scattered to the children of a 2x subdivision: with cout > 0, the conv's output
 // channel c = o * cout + k of row i goes to row mstart[i] + (octants of parent i kept before o)
 // of an [M][cout] output when mask[8 i + o] != 0, and nowhere otherwise (the octant gather of
@@ -96,32 +107,39 @@ struct OctantScatter {
     // parent of 32-row block b of that row group keeps octant o. The MFMAs of a block whose
     // parents keep none of a wave's octant are skipped: those outputs are never stored.
     const uint32_t* blocks = nullptr;
-    // Optional, an octant plan (octant_plan_build; its tiles are the `plan` argument then): *oct_tiles
-    // tiles of each octant, oct_cap at most, tile k of octant o at 8 k + o; cout % 128 == 0. Every
-    // MFMA then works for a row that is stored, where with `blocks` a block of 32 parents is rarely
-    // without one that keeps the octant. The sums are the same bits.
-    const int32_t* oct_tiles = nullptr;
+    // Optional, an octant plan (octant_plan_build): its state, and its oct_cap tiles at oct_plan;
+    // cout % 128 == 0. The kernels run on it where the state says so (octant_taken: known on the
+    // device only), otherwise on the `plan` argument with `blocks`. On the octant plan every MFMA
+    // works for a row that is stored, where a block of 32 parents is rarely without one that keeps the
+    // octant. The sums are the same bits. side: a launch that runs on one of the two plans only.
+    const OctantTiles* oct = nullptr;
+    void* oct_plan = nullptr;
     int oct_cap = 0;
+    enum Side { EITHER, OCTANTS, PARENTS } side = EITHER;
 };
 
-// An octant plan: for each octant, the parents that keep it as tiles of `rows` parents in the order
-// of the plan's walk, with their own distinct rows, slots and act bits. The octants' tiles take
-// turns, so that the units running together on an XCD share feature rows: with an octant's tiles
-// in a row instead, each XCD streamed every feature row (256 -> 128 at 60 K parents: 1100 us).
+// An octant plan: for each octant, the parents that keep it as tiles of their own in the order of
+// the plan's walk, with their own distinct rows, slots and act bits. The conv lets the octants'
+// tiles take turns, so that the units running together on an XCD share feature rows: with an
+// octant's tiles in a row instead, each XCD streamed every feature row (256 -> 128 at 60 K parents:
+// 1100 us).
 struct OctantPlan {
-    int rows = 0;         // parents of a tile (a multiple of 32 up to HB_M)
-    int cap = 0;          // tiles of an octant, at most
+    int cap = 0;          // tiles, at most
+    // The conv's time in rounds of units, in tenths: on the parents' plan base_cost, on the octant plan
+    // 10 ceil(ceil(T mul / 8) / fit) for T tiles of the octant that has most (by_sum: of all octants).
+    int base_cost = 0, mul = 0, fit = 0;
+    bool by_sum = false;
     size_t plan_bytes = 0, member_bytes = 0, count_bytes = 0;
 };
-// Whether conv1 of n parents and m children (cin -> 8 cout) takes an octant plan, and its sizes.
+// Whether conv1 of n parents and m children (cin -> 8 cout) may take an octant plan, and its sizes.
 bool octant_plan_spec(int64_t n, int64_t m, int cin, int cout, OctantPlan& op);
-// Builds it from the parents' stored plan, table and mask: tiles into oplan (op.plan_bytes); members
-// and counts are scratch; *oct_tiles: the tiles of the octant that has most.
+// Builds it from the parents' stored plan, table and mask: tiles into oplan (op.plan_bytes), state
+// into *oct; members and counts are scratch. blocks: as octant_blocks writes them.
 int octant_plan_build(const OctantPlan& op, const void* plan, int64_t n, const int32_t* nbr, const uint8_t* mask,
-                      void* oplan, int32_t* members, int32_t* counts, int32_t* oct_tiles, hipStream_t s);
+                      void* oplan, int32_t* members, int32_t* counts, uint32_t* blocks, OctantTiles* oct, hipStream_t s);
 
-// The words OctantScatter::blocks reads, for a stored plan of n parents and their mask [8 n]:
-// out [n_tiles * 4].
+// The words OctantScatter::blocks reads, for a stored plan of n parents and their mask [8 n] (8-byte
+// aligned): out [n_tiles * 4].
 int octant_blocks(const void* plan, int64_t n, const uint8_t* mask, uint32_t* out, hipStream_t s);
 
 // The C2S skip added by the conv's stores (sparse.cpp:302-323): with cin > 0, output row m
@@ -179,6 +197,8 @@ int64_t column_split_tiles(int64_t n_tiles, int nct, int cus);
 // the stores that need 128 whole channels, else 1). A rule on sizes alone: with and without a plan,
 // and over any tiles of it, a conv takes the same kernel and sums in the same order.
 int conv_split_pick(int64_t n, int ci, int co, int ncg);
+// Compute units of the current device.
+int conv_cus();
 
 // tr (planned only): the plan's tiles to run, all of them by default; a narrower range runs in one
 // launch of its units.
@@ -187,11 +207,9 @@ int halo_conv_launch(int fdt, int odt, const void* feats, int64_t n, int ci, con
                      hipStream_t s, OctantScatter osc = {}, SkipAdd skip = {}, PadRow pad = {},
                      RowNorm ln = {}, TileRange tr = {});
 
-// tsp_subm_conv3x3_planned_octants with, when blocks is not null, the MFMAs of row blocks whose
-// parents keep none of a wave's octant skipped (blocks from octant_blocks).
+// tsp_subm_conv3x3_planned_octants with all of osc's options.
 int planned_octants(const void* feats, int dtype, int64_t n, int ci, const int32_t* nbr, const void* plan,
-                    const void* packed, const float* bias, int cout, const uint8_t* mask, const int32_t* mstart,
-                    float* out, const uint32_t* blocks, hipStream_t s);
+                    const void* packed, const float* bias, const OctantScatter& osc, float* out, hipStream_t s);
 
 // tsp_subm_conv3x3_planned_skip with, when out16 is not null, out also rounded to out16_dtype
 // (TSP_BF16 or TSP_F16) in out16 [n][co] by the same stores.

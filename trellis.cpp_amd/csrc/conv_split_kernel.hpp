@@ -57,18 +57,37 @@ __global__ __launch_bounds__(512, 1) void k_conv_split(
     // few weight columns, in tile-major order on few feature rows: the caller picks by which is
     // larger, the weights or the features.
     constexpr bool OCT = EPI == 1 || EPI == 4 || EPI == 5;
+    int64_t units = n_tiles * n_ctiles * RS;
+    bool on_oct = false;
     if constexpr (EPI == 1 || EPI == 5) {
-        if (osc.oct_tiles) {   // an octant plan: its tile count is known on the device only
-            n_tiles = min<int64_t>(n_tiles, *osc.oct_tiles);
-            per_xcd = (n_tiles * n_ctiles * RS + 7) / 8;
+        if (!octant_side(osc, plan)) return;
+        if (osc.oct) {   // (never more units than on the parents' plan)
+            on_oct = true;
+            units = (int64_t)osc.oct->total * (osc.cout / BN) * RS;
+            per_xcd = (units + 7) / 8;
         }
     }
-    const int64_t units = n_tiles * n_ctiles * RS;
     const int64_t u = (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (blockIdx.x / 8 >= per_xcd || u >= units) return;
     int64_t tile;
     int ct, rsub;
-    if (ctile_major) {
+    if (on_oct) {
+        // octant after octant in column-tile-major order; otherwise the octants take turns
+        const int cpo = osc.cout / BN;               // column tiles of an octant
+        rsub = (int)(u % RS);
+        int oct, k, c;
+        if (ctile_major) {
+            int64_t v = u / RS;
+            for (oct = 0; oct < 7 && v >= (int64_t)osc.oct->tiles[oct] * cpo; ++oct) v -= (int64_t)osc.oct->tiles[oct] * cpo;
+            c = (int)(v / osc.oct->tiles[oct]);
+            k = (int)(v % osc.oct->tiles[oct]);
+        } else {
+            c = (int)(u / RS % cpo);
+            octant_turn(osc.oct, (int)(u / RS / cpo), oct, k);
+        }
+        tile = osc.oct->base[oct] + k;
+        ct = oct * cpo + c;
+    } else if (ctile_major) {
         const int64_t pc = n_tiles * RS;
         ct = (int)(u / pc);
         tile = (u % pc) / RS;
@@ -78,9 +97,6 @@ __global__ __launch_bounds__(512, 1) void k_conv_split(
         const int k = (int)(u % ((int64_t)n_ctiles * RS));
         ct = k / RS;
         rsub = k % RS;
-    }
-    if constexpr (EPI == 1 || EPI == 5) {
-        if (osc.oct_tiles) tile = tile * 8 + ct * BN / osc.cout;   // tile k of octant o: 8 k + o
     }
     const int64_t row0 = tile * HB_M;
 
@@ -558,7 +574,7 @@ int split_launch(int odt, bool planned, const void* feats, int64_t n, int ci, co
                  SkipAdd skip, PadRow pad, RowNorm ln, TileRange tr) {
     constexpr int BN = 64 * NCG;
     constexpr int O16 = BF16 ? TSP_BF16 : TSP_F16;
-    const int64_t all_tiles = osc.oct_tiles ? osc.oct_cap : ceil_div(n, HB_M);   // (an octant plan: of each octant)
+    const int64_t all_tiles = ceil_div(n, HB_M);
     const int64_t t0 = planned ? tr.t0 : 0;
     const int64_t n_tiles = planned && tr.nt >= 0 ? tr.nt : all_tiles - t0;
     if (t0 < 0 || n_tiles < 0 || t0 + n_tiles > all_tiles) {
@@ -572,7 +588,7 @@ int split_launch(int odt, bool planned, const void* feats, int64_t n, int ci, co
     const bool ctile_major = n < (int64_t)kTaps * co;
     PlanView pv{};
     if (planned) {
-        pv = carve_plan(const_cast<void*>(plan), osc.oct_tiles ? 8 * all_tiles : all_tiles);
+        pv = carve_plan(const_cast<void*>(plan), all_tiles);
         pv.hdr += t0 * 4;
         pv.rowof += t0 * HB_SLOTS;
         pv.slots += t0 * HB_SLOT_TABLE;

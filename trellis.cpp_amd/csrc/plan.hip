@@ -603,13 +603,10 @@ __global__ __launch_bounds__(HB_PLAN_NT) __attribute__((amdgpu_waves_per_eu(6)))
     for (int t = 0; t < kTaps; ++t) sl[t * HB_M] = (uint16_t)(wsl[t >> 1] >> (16 * (t & 1)));
 }
 
-// The voxels of an octant plan's tiles: tile k of octant o is tile q = 8 k + o, its voxels
-// members[HB_M q ..], `rows` of them at most, of the octant's totals[o]; *tiles tiles an octant.
+// The voxels of an octant plan's tiles: tile q's at members[HB_M q ..].
 struct OctantMembers {
     const int32_t* members = nullptr;
-    const int32_t* tiles = nullptr;
-    const int32_t* totals = nullptr;
-    int rows = 0;
+    OctantTiles* oct = nullptr;
 };
 
 // Tiles ranked from the table's entries: tiles list[0 .. *list_n) (cell walk order when the grid is
@@ -632,13 +629,16 @@ __global__ __launch_bounds__(HB_PLAN_NT) __attribute__((amdgpu_waves_per_eu(4)))
     __shared__ uint32_t sAct[4 * HB_ACT_WORDS];
     const int tid = threadIdx.x;
     const bool walk = order != nullptr && hdr->mode == GRID_MODE_CELLS;
-    const int64_t count = list ? (int64_t)*list_n : om.members ? min<int64_t>(8 * (int64_t)*om.tiles, n_tiles) : n_tiles;
+    const int64_t count = list ? (int64_t)*list_n : om.members ? (om.oct->fits ? (int64_t)om.oct->total : 0) : n_tiles;
     for (int64_t k = blockIdx.x; k < count; k += gridDim.x) {
         const int64_t tile = list ? (int64_t)list[k] : k;
         const int64_t q = tile * HB_M + tid;
         int64_t i[1];
         if (om.members) {
-            i[0] = tid < om.rows && (tile >> 3) * om.rows + tid < om.totals[tile & 7] ? (int64_t)om.members[q] : -1;
+            int o = 0;
+            while (o < 7 && tile >= om.oct->base[o] + om.oct->tiles[o]) ++o;
+            const int rows = om.oct->rows[o];
+            i[0] = tid < rows && (tile - om.oct->base[o]) * rows + tid < om.oct->count[o] ? (int64_t)om.members[q] : -1;
         } else {
             i[0] = q < n ? (walk ? (int64_t)order[q] : q) : -1;
         }
@@ -654,6 +654,7 @@ __global__ __launch_bounds__(HB_PLAN_NT) __attribute__((amdgpu_waves_per_eu(4)))
         if (tid == 0) {
             int32_t* h = plan.hdr + tile * 4;
             h[0] = H; h[1] = direct ? 1 : 0; h[2] = 0; h[3] = 0;
+            if (om.members && direct) atomicAdd(&om.oct->direct, 1);
         }
         if (!direct) {
             int32_t* ro = plan.rowof + tile * HB_SLOTS;
@@ -676,58 +677,102 @@ __device__ __forceinline__ uint32_t kept_octants(const uint8_t* __restrict__ mas
     return kept;
 }
 
-// counts[o n_tiles + tile] = the parents of plan tile `tile` that keep octant o.
+// A workgroup a plan tile, a thread a position. counts (optional): counts[o n_tiles + tile] = the
+// parents of the tile that keep octant o. blocks: the octants each position's parent keeps, ORed over
+// each 32-position block (a wave's ballot covers two) into the word of its row group: bit 4 o + b for
+// block b (0..3) of the 128 positions of row group p / 128.
 __global__ __launch_bounds__(HB_M) void k_octant_count(const int32_t* __restrict__ vox, int64_t n,
                                                        const uint8_t* __restrict__ mask, int64_t n_tiles,
-                                                       int32_t* __restrict__ counts) {
+                                                       int32_t* __restrict__ counts, uint32_t* __restrict__ blocks) {
     __shared__ int sC[8];
-    const int tid = threadIdx.x;
+    __shared__ uint32_t sB[HB_M / 128];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (tid < 8) sC[tid] = 0;
+    if (tid < HB_M / 128) sB[tid] = 0u;
     __syncthreads();
     const int32_t v = vox[(int64_t)blockIdx.x * HB_M + tid];
     const uint32_t kept = v >= 0 && v < n ? kept_octants(mask, v) : 0u;
+    uint32_t bits = 0;
+    const int b0 = (wave & 1) * 2;   // this wave's first block within its row group
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
         const uint64_t b = __ballot((kept >> o) & 1u);
-        if ((tid & 63) == 0 && b) atomicAdd(&sC[o], __popcll(b));
+        bits |= ((uint32_t)b != 0u ? 1u : 0u) << (4 * o + b0);
+        bits |= ((uint32_t)(b >> 32) != 0u ? 1u : 0u) << (4 * o + b0 + 1);
+        if (counts && lane == 0 && b) atomicAdd(&sC[o], __popcll(b));
     }
+    if (lane == 0 && bits) atomicOr(&sB[wave >> 1], bits);
     __syncthreads();
-    if (tid < 8) counts[tid * n_tiles + blockIdx.x] = sC[tid];
+    if (counts && tid < 8) counts[tid * n_tiles + blockIdx.x] = sC[tid];
+    if (tid < HB_M / 128) blocks[(int64_t)blockIdx.x * (HB_M / 128) + tid] = sB[tid];
 }
 
+// A tile's parents span at most this many voxels of the walk: they stage up to HB_SLOTS distinct
+// rows, 1.4 a voxel on bands, up to 1.7 (at 1216, 2 of 508 tiles were past them where four octants are
+// kept by 35 %).
+constexpr int OCT_SPAN = 1152;
+
 // One workgroup, 128 threads an octant: the counts' exclusive prefixes over the tiles, in place; then
-// the octants' totals and the most tiles of one.
-__global__ __launch_bounds__(1024) void k_octant_scan(int64_t n_tiles, int rows, int32_t* __restrict__ counts,
-                                                      int32_t* __restrict__ totals, int32_t* __restrict__ oct_tiles) {
-    __shared__ int sS[1024];
-    __shared__ int sT[8];
-    const int tid = threadIdx.x, o = tid >> 7, t = tid & 127;
+// each octant's tiles, and whether the plan is taken: where its tiles fit the space and its rounds of
+// units are a tenth fewer than the parents' plan's. A unit costs about the same on either, however
+// many of its MFMAs are skipped, and a workgroup of the large-grid kernel keeps its octant, so the
+// fullest octant decides there. 60 K 256 -> 128, us up to conv2 on the octant plan and on the parents':
+// every octant kept by 27 % 360 and 708, by 75 % 631 and 706; one octant by all and seven by 5 % (not
+// taken, some 15 us for the build's launches) 741 and 671 -- with the mean's tiles for every octant it
+// took 4085. A tile whose rows are read from memory runs eight times as long, on either plan: seven
+// rounds more for its workgroup.
+__global__ __launch_bounds__(1024) void k_octant_scan(int64_t n, int64_t n_tiles, const int32_t* __restrict__ hdr,
+                                                      OctantPlan op, int32_t* __restrict__ counts,
+                                                      OctantTiles* __restrict__ oct) {
+    __shared__ int sW[16];
+    __shared__ OctantTiles sO;
+    __shared__ int sD;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, o = tid >> 7, t = tid & 127;
     const int64_t chunk = (n_tiles + 127) / 128, b = t * chunk, e = min<int64_t>(n_tiles, b + chunk);
     int32_t* c = counts + o * n_tiles;
     int sum = 0;
     for (int64_t k = b; k < e; ++k) sum += c[k];
-    sS[tid] = sum;
-    __syncthreads();
-    int before = 0, all = 0;
-    for (int k = 0; k < 128; ++k) {
-        const int v = sS[(o << 7) + k];
-        before += k < t ? v : 0;
-        all += v;
+    int direct = 0;
+    for (int64_t k = tid; k < n_tiles; k += 1024) direct += hdr[4 * k + 1] != 0;
+    int before = sum;   // inclusive over the wave, then exclusive over the octant's two waves
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(before, off, 64);
+        if (lane >= off) before += y;
     }
+    if (lane == 63) sW[wave] = before;
+    if (tid == 0) sD = 0;
+    __syncthreads();
+    if (direct) atomicAdd(&sD, direct);
+    before += (wave & 1 ? sW[wave - 1] : 0) - sum;
     for (int64_t k = b; k < e; ++k) {
         const int v = c[k];
         c[k] = before;
         before += v;
     }
-    if (t == 0) sT[o] = all;
+    if (tid < 8) {
+        const int all = sW[2 * tid] + sW[2 * tid + 1];
+        const int rows = (int)min<int64_t>(HB_M, (int64_t)OCT_SPAN * all / n);
+        sO.rows[tid] = max(rows / 8 * 8, 16);
+        sO.count[tid] = all;
+        sO.tiles[tid] = (all + sO.rows[tid] - 1) / sO.rows[tid];
+    }
     __syncthreads();
     if (tid == 0) {
-        int most = 0;
+        int total = 0, most = 0;
         for (int k = 0; k < 8; ++k) {
-            totals[k] = sT[k];
-            most = max(most, sT[k]);
+            sO.base[k] = total;
+            total += sO.tiles[k];
+            most = max(most, sO.tiles[k]);
         }
-        *oct_tiles = (most + rows - 1) / rows;
+        const int64_t units = ((op.by_sum ? total : most) * (int64_t)op.mul + 7) / 8;
+        const int64_t cost = 10 * ((units + op.fit - 1) / op.fit), base = op.base_cost + (sD ? 70 : 0);
+        // (the launch's grid is the parents' tiles')
+        sO.fits = total <= op.cap && total <= 8 * n_tiles && most <= n_tiles && 10 * cost <= 9 * base;
+        sO.spare = base - cost >= 160 ? total / 128 : base - cost >= 80 ? 1 : 0;
+        sO.direct = 0;
+        sO.total = total;
+        sO.most = most;
+        *oct = sO;
     }
 }
 
@@ -737,11 +782,13 @@ __global__ __launch_bounds__(1024) void k_octant_scan(int64_t n_tiles, int rows,
 // own positions, grouped by corner taps, the cut is scattered over the patch: 1750-1870 distinct rows
 // a tile instead of 1440-1500 on bands, and 4-16 % of the tiles past HB_SLOTS.
 __global__ __launch_bounds__(HB_M) void k_octant_members(const int32_t* __restrict__ vox, int64_t n,
-                                                         const uint8_t* __restrict__ mask, int64_t n_tiles, int rows,
-                                                         int cap, const int32_t* __restrict__ counts,
+                                                         const uint8_t* __restrict__ mask, int64_t n_tiles,
+                                                         const OctantTiles* __restrict__ oct,
+                                                         const int32_t* __restrict__ counts,
                                                          int32_t* __restrict__ members) {
     __shared__ int sW[8][HB_M / 64];
     __shared__ uint32_t sV[HB_M];
+    if (!oct->fits) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     sV[tid] = (uint32_t)vox[(int64_t)blockIdx.x * HB_M + tid];   // (-1, no voxel, sorts last)
     __syncthreads();
@@ -772,7 +819,8 @@ __global__ __launch_bounds__(HB_M) void k_octant_members(const int32_t* __restri
         if (!((kept >> o) & 1u)) continue;
         int r = counts[o * n_tiles + blockIdx.x] + before[o];
         for (int w = 0; w < wave; ++w) r += sW[o][w];
-        if (r / rows < cap) members[((int64_t)(r / rows) * 8 + o) * HB_M + r % rows] = v;
+        const int rows = oct->rows[o];
+        members[((int64_t)oct->base[o] + r / rows) * HB_M + r % rows] = v;
     }
 }
 
@@ -781,45 +829,63 @@ __global__ __launch_bounds__(HB_M) void k_octant_members(const int32_t* __restri
 bool octant_plan_spec(int64_t n, int64_t m, int cin, int cout, OctantPlan& op) {
     // Half of the octants are kept on a surface band (m = 4.1 n), so the plan halves conv1; its build
     // costs 40-60 us up to 100 K parents. Taken where conv1 is long enough to pay (150 us at the rate
-    // of the full conv), where it leaves out a fifth of the work at least, and where the kernel's
+    // of the full conv), where it may leave out a fifth of the work at least, and where the kernel's
     // 128-column tiles lie in one octant. The C2S block, us with and without: 60 K 256 -> 128 642 and
-    // 890; 12 K 512 -> 256 525 and 717; 33.5 K 1024 -> 512 4990 and 7260.
+    // 890; 12 K 512 -> 256 525 and 717; 33.5 K 1024 -> 512 4990 and 7260. Whether the octants' own
+    // counts bear it out is decided on the device (k_octant_scan).
     if (cout % 128 != 0 || n <= 0 || m <= 0) return false;
-    const double pay = conv_split_pick(n, cin, 8 * cout, cout == 128 ? 2 : 1) ? 7e8 : 4.3e8;   // (idle CUs: less to win)
-    if ((double)n * cin * cout < pay || 10 * m > 64 * n) return false;
-    // A tile's parents span rows / (m / 8n) voxels of the walk, which stage at most HB_SLOTS distinct
-    // rows: 1.4 rows a voxel on bands, up to 1.7.
-    const int64_t rows = std::min<int64_t>(HB_M, 1216 * m / (8 * n) / 32 * 32);
+    const int co = 8 * cout, ncg = cout == 128 ? 2 : 1, cus = conv_cus();
+    const int rgw = conv_split_pick(n, cin, co, ncg);
+    if ((double)n * cin * cout < (rgw ? 7e8 : 4.3e8) || 10 * m > 64 * n) return false;   // (idle CUs: less to win)
+    const int64_t rows = std::min<int64_t>(HB_M, OCT_SPAN * m / (8 * n) / 32 * 32);
     if (rows < 192) return false;
-    const int64_t cap = ceil_div(std::min(n, m), rows), tiles = ceil_div(n, HB_M);   // (every parent keeps an octant)
+    // room for the tiles of evenly kept octants and a tenth more; more tiles would win little
+    const int64_t cap = 11 * ceil_div(m, rows) / 10 + 16, tiles = ceil_div(n, HB_M);
     if (cap > INT32_MAX / 16) return false;
-    op.rows = (int)rows;
     op.cap = (int)cap;
-    op.plan_bytes = plan_tile_bytes(8 * cap);
-    op.member_bytes = (size_t)cap * 8 * HB_M * 4;
-    op.count_bytes = ((size_t)tiles * 8 + 8) * 4;
+    if (rgw) {   // the units of all octants' tiles, any compute unit
+        op.by_sum = true;
+        op.mul = cout / (64 * ncg) * (4 / rgw);
+        op.fit = std::max(1, cus / 8);
+        op.base_cost = (int)(10 * ceil_div(ceil_div(8 * tiles * op.mul, 8), op.fit));
+    } else {     // a workgroup keeps its column, so its octant
+        op.by_sum = false;
+        op.mul = co / 128;
+        op.fit = std::max(1, cus / 8 / op.mul) * op.mul;
+        const int64_t split = cout == 128 ? 0 : column_split_tiles(tiles, op.mul, cus);   // (a thin last round: 0.65)
+        op.base_cost = (int)(10 * ceil_div(ceil_div((split ? split : tiles) * op.mul, 8), op.fit) + (split ? 6 : 0));
+    }
+    op.plan_bytes = plan_tile_bytes(cap);
+    op.member_bytes = (size_t)cap * HB_M * 4;
+    op.count_bytes = (size_t)tiles * 8 * 4;
     return true;
 }
 
+int octant_blocks(const void* plan, int64_t n, const uint8_t* mask, uint32_t* out, hipStream_t s) {
+    const int64_t n_tiles = ceil_div(n, HB_M);
+    if (n_tiles == 0) return TSP_OK;
+    const PlanView pv = carve_plan(const_cast<void*>(plan), n_tiles);
+    hipLaunchKernelGGL(k_octant_count, dim3((unsigned)n_tiles), dim3(HB_M), 0, s, pv.vox, n, mask, n_tiles, nullptr, out);
+    TSP_CHECK_LAUNCH();
+    return TSP_OK;
+}
+
 int octant_plan_build(const OctantPlan& op, const void* plan, int64_t n, const int32_t* nbr, const uint8_t* mask,
-                      void* oplan, int32_t* members, int32_t* counts, int32_t* oct_tiles, hipStream_t s) {
+                      void* oplan, int32_t* members, int32_t* counts, uint32_t* blocks, OctantTiles* oct, hipStream_t s) {
     const int64_t tiles = ceil_div(n, HB_M);
     const PlanView pv = carve_plan(const_cast<void*>(plan), tiles);
-    int32_t* totals = counts + 8 * tiles;
-    hipLaunchKernelGGL(k_octant_count, dim3((unsigned)tiles), dim3(HB_M), 0, s, pv.vox, n, mask, tiles, counts);
+    hipLaunchKernelGGL(k_octant_count, dim3((unsigned)tiles), dim3(HB_M), 0, s, pv.vox, n, mask, tiles, counts, blocks);
     TSP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_octant_scan, dim3(1), dim3(1024), 0, s, tiles, op.rows, counts, totals, oct_tiles);
+    hipLaunchKernelGGL(k_octant_scan, dim3(1), dim3(1024), 0, s, n, tiles, pv.hdr, op, counts, oct);
     TSP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_octant_members, dim3((unsigned)tiles), dim3(HB_M), 0, s, pv.vox, n, mask, tiles, op.rows,
-                       op.cap, counts, members);
+    hipLaunchKernelGGL(k_octant_members, dim3((unsigned)tiles), dim3(HB_M), 0, s, pv.vox, n, mask, tiles, oct, counts,
+                       members);
     TSP_CHECK_LAUNCH();
     OctantMembers om;
     om.members = members;
-    om.tiles = oct_tiles;
-    om.totals = totals;
-    om.rows = op.rows;
-    hipLaunchKernelGGL(k_plan_table, dim3((unsigned)std::min(8 * op.cap, 4096)), dim3(HB_PLAN_NT), 0, s, nbr, n, nullptr,
-                       nullptr, nullptr, nullptr, (int64_t)8 * op.cap, carve_plan(oplan, 8 * (int64_t)op.cap), om);
+    om.oct = oct;
+    hipLaunchKernelGGL(k_plan_table, dim3((unsigned)std::min(op.cap, 4096)), dim3(HB_PLAN_NT), 0, s, nbr, n, nullptr,
+                       nullptr, nullptr, nullptr, (int64_t)op.cap, carve_plan(oplan, op.cap), om);
     TSP_CHECK_LAUNCH();
     return TSP_OK;
 }

@@ -46,7 +46,7 @@ struct PlanView {
     int32_t* vox;
     uint32_t* act;
 };
-inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
+__host__ __device__ inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 __host__ __device__ inline PlanView carve_plan(void* p, int64_t n_tiles) {
     char* c = reinterpret_cast<char*>(p);
     PlanView v;
@@ -60,6 +60,43 @@ __host__ __device__ inline PlanView carve_plan(void* p, int64_t n_tiles) {
     c += align256((size_t)n_tiles * HB_M * 4);
     v.act = reinterpret_cast<uint32_t*>(c);
     return v;
+}
+// Whether conv1 runs on the octant plan (its build is done).
+__device__ __forceinline__ bool octant_taken(const OctantTiles* t) { return t->fits && t->direct <= t->spare; }
+// The plan a launch runs on: with an octant plan taken, plan becomes it, without its block words;
+// else osc.oct becomes null. False when the launch is for the other one.
+__device__ __forceinline__ bool octant_side(OctantScatter& osc, PlanView& plan) {
+    if (!osc.oct) return true;
+    const bool taken = octant_taken(osc.oct);
+    if (taken ? osc.side == OctantScatter::PARENTS : osc.side == OctantScatter::OCTANTS) return false;
+    if (taken) {
+        plan = carve_plan(osc.oct_plan, osc.oct_cap);
+        osc.blocks = nullptr;
+    } else {
+        osc.oct = nullptr;
+    }
+    return true;
+}
+// Tile q (< t->total) of an octant plan where the octants' tiles take turns: tile k of octant o.
+__device__ __forceinline__ void octant_turn(const OctantTiles* t, int q, int& o, int& k) {
+    o = k = 0;
+    for (int k0 = 0, pass = 0; pass < 8; ++pass) {
+        int octants = 0, next = INT32_MAX;   // the octants with tiles from k0 on; the first end among them
+        for (int i = 0; i < 8; ++i)
+            if (t->tiles[i] > k0) {
+                ++octants;
+                next = min(next, t->tiles[i]);
+            }
+        if (octants == 0) return;
+        if ((int64_t)q < (int64_t)(next - k0) * octants) {
+            k = k0 + q / octants;
+            for (int j = q % octants; o < 7; ++o)
+                if (t->tiles[o] > k0 && j-- == 0) break;
+            return;
+        }
+        q -= (next - k0) * octants;
+        k0 = next;
+    }
 }
 // bytes of the tile records (without the build's sort scratch)
 inline size_t plan_tile_bytes(int64_t n_tiles) {
