@@ -120,8 +120,10 @@ __global__ __launch_bounds__(GB_NT) void k_grid_clear(const int32_t* __restrict_
     }
     __syncthreads();
     if (sH.mode != GRID_MODE_CELLS) return;
-    const int64_t nw = sH.dir_n;
-    for (int64_t i = blockIdx.x * (int64_t)GB_NT + tid; i < nw; i += (int64_t)gridDim.x * GB_NT) dir[i] = 0;
+    // (up to 3 words past the directory: the blocks start at a multiple of 64)
+    u32x4_t* d4 = reinterpret_cast<u32x4_t*>(dir);
+    const int64_t n4 = (sH.dir_n + 3) / 4;
+    for (int64_t i = blockIdx.x * (int64_t)GB_NT + tid; i < n4; i += (int64_t)gridDim.x * GB_NT) d4[i] = u32x4_t{0u, 0u, 0u, 0u};
 }
 
 __global__ __launch_bounds__(GB_NT) void k_grid_mark(const int32_t* __restrict__ coords, int64_t n,
@@ -144,16 +146,29 @@ __global__ __launch_bounds__(GB_NT) void k_grid_mark(const int32_t* __restrict__
     }
 }
 
-// Occupied directory words of each of np chunks into parts[].
+// The four directory words of a thread from word i (a multiple of 4): bit k set where word i + k is
+// occupied and before e.
+__device__ __forceinline__ uint32_t occupied4(const int32_t* __restrict__ dir, int64_t i, int64_t e) {
+    if (i >= e) return 0u;
+    const u32x4_t w = *reinterpret_cast<const u32x4_t*>(dir + i);
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) m |= (w[k] != 0u && i + k < e ? 1u : 0u) << k;
+    return m;
+}
+
+// Occupied directory words of each of dir_parts chunks into parts[].
 __global__ __launch_bounds__(GB_NT) void k_grid_scan(const GridHdr* __restrict__ hdr, const int32_t* __restrict__ dir,
-                                                     int32_t* __restrict__ parts, int np) {
+                                                     int32_t* __restrict__ parts) {
     __shared__ int sW[GB_NT / 64];
     if (hdr->mode != GRID_MODE_CELLS) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int64_t nw = hdr->dir_n, chunk = (nw + np - 1) / np;
-    const int64_t b = blockIdx.x * chunk, e = min(nw, b + chunk);
+    const int64_t nw = hdr->dir_n;
+    const int np = dir_parts(nw, gridDim.x);
+    if ((int)blockIdx.x >= np) return;
+    const int64_t chunk = dir_chunk(nw, np), b = blockIdx.x * chunk, e = min(nw, b + chunk);
     int c = 0;
-    for (int64_t i = b + tid; i < e; i += GB_NT) c += dir[i] != 0;
+    for (int64_t i = b + 4 * tid; i < e; i += DIR_WORDS) c += __popc(occupied4(dir, i, e));
     c = wave_sum_i(c);
     if (lane == 0) sW[wave] = c;
     __syncthreads();
@@ -164,15 +179,14 @@ __global__ __launch_bounds__(GB_NT) void k_grid_scan(const GridHdr* __restrict__
     }
 }
 
-// Every workgroup sums the np partials for its own prefix and the block count, and
-// decides whether the blocks fit the region and the caller's block_cap (the same answer in each;
+// Every workgroup sums the partials for its own prefix and the block count, and decides whether the blocks fit the region and the caller's block_cap (the same answer in each;
 // workgroup 0 records it). Then: block
 // numbers into the directory (Morton order; cell_of, when given, gets each block's directory
 // index) and the blocks cleared; or, when the grid does not fit and a hash is given, the hash's
 // buckets cleared.
 __global__ __launch_bounds__(GB_NT) void k_grid_apply(GridHdr* __restrict__ hdr, int32_t* __restrict__ dir,
                                                       const int32_t* __restrict__ parts, HashView hash,
-                                                      int32_t* __restrict__ cell_of, int64_t block_cap, int np) {
+                                                      int32_t* __restrict__ cell_of, int64_t block_cap) {
     __shared__ int sW[2][GB_NT / 64];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     // Read once a workgroup: workgroup 0 may write the fallback while another one starts, which then
@@ -181,6 +195,8 @@ __global__ __launch_bounds__(GB_NT) void k_grid_apply(GridHdr* __restrict__ hdr,
     if (tid == 0) sMode = hdr->mode;
     __syncthreads();
     bool cells = sMode == GRID_MODE_CELLS;
+    const int64_t nw = hdr->dir_n;
+    const int np = dir_parts(nw, gridDim.x);
     int64_t nblocks = 0;
     int run = 0;
     if (cells) {
@@ -214,23 +230,32 @@ __global__ __launch_bounds__(GB_NT) void k_grid_apply(GridHdr* __restrict__ hdr,
             w[s] = u32x4_t{0u, 0u, 0u, 0u};
         return;
     }
-    const int64_t nw = hdr->dir_n, chunk = (nw + np - 1) / np;
-    const int64_t b = blockIdx.x * chunk, e = min(nw, b + chunk);
-    for (int64_t r0 = b; r0 < e; r0 += GB_NT) {
-        const int64_t i = r0 + tid;
-        const bool occ = i < e && dir[i] != 0;
-        const uint64_t bal = __ballot(occ);
-        if (lane == 0) sW[0][wave] = __popcll(bal);
+    const int64_t chunk = dir_chunk(nw, np), b = blockIdx.x * chunk, e = min(nw, b + chunk);   // (no words past np)
+    for (int64_t r0 = b; r0 < e; r0 += DIR_WORDS) {
+        const int64_t i = r0 + 4 * tid;
+        const uint32_t occ = occupied4(dir, i, e);
+        const uint64_t below = (1ull << lane) - 1ull;
+        int mine = 0, all = 0;   // occupied words of the wave's lower lanes, of the wave
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint64_t bal = __ballot((occ >> k) & 1u);
+            mine += __popcll(bal & below);
+            all += __popcll(bal);
+        }
+        if (lane == 0) sW[0][wave] = all;
         __syncthreads();
         int before = 0, total = 0;
         for (int w = 0; w < GB_NT / 64; ++w) {
             if (w < wave) before += sW[0][w];
             total += sW[0][w];
         }
-        if (occ) {
-            const int id = run + before + __popcll(bal & ((1ull << lane) - 1ull));
-            dir[i] = id + 1;
-            if (cell_of) cell_of[id] = (int32_t)i;
+        int id = run + before + mine;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (!((occ >> k) & 1u)) continue;
+            dir[i + k] = id + 1;
+            if (cell_of) cell_of[id] = (int32_t)(i + k);
+            ++id;
         }
         run += total;
         __syncthreads();
@@ -305,19 +330,19 @@ int grid_build(const int32_t* coords, int64_t n, void* region, size_t region_byt
                int32_t* status, HashView hash, int32_t* cell_of, int64_t block_cap, hipStream_t s) {
     const GridTail gt = carve_grid_tail(tail);
     int32_t* dir = static_cast<int32_t*>(region);
-    const unsigned np = (unsigned)grid_parts(n);
+    const unsigned np = (unsigned)grid_parts(n), nd = (unsigned)grid_workgroups(n);
     const unsigned nvb = (unsigned)std::max<int64_t>(1, ceil_div(n, GB_NT));
     hipLaunchKernelGGL(k_grid_bbox, dim3(np), dim3(GB_NT), 0, s, coords, n, gt.parts, status);
     TSP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_grid_clear, dim3(np), dim3(GB_NT), 0, s, gt.parts, gt.hdr, dir,
+    hipLaunchKernelGGL(k_grid_clear, dim3(nd), dim3(GB_NT), 0, s, gt.parts, gt.hdr, dir,
                        (int64_t)(region_bytes / 4), (int)np);
     TSP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_grid_mark, dim3(nvb), dim3(GB_NT), 0, s, coords, n, gt.hdr, dir);
     TSP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_grid_scan, dim3(np), dim3(GB_NT), 0, s, gt.hdr, dir, gt.parts, (int)np);
+    hipLaunchKernelGGL(k_grid_scan, dim3(nd), dim3(GB_NT), 0, s, gt.hdr, dir, gt.parts);
     TSP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_grid_apply, dim3(np), dim3(GB_NT), 0, s, gt.hdr, dir, gt.parts, hash, cell_of,
-                       block_cap, (int)np);
+    hipLaunchKernelGGL(k_grid_apply, dim3(nd), dim3(GB_NT), 0, s, gt.hdr, dir, gt.parts, hash, cell_of,
+                       block_cap);
     TSP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_grid_insert, dim3(nvb), dim3(GB_NT), 0, s, coords, n, gt.hdr, dir, hash);
     TSP_CHECK_LAUNCH();

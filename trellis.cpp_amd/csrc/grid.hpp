@@ -27,12 +27,32 @@ constexpr int GRID_MAX_BITS = 10;              // directory of at most 2^30 cell
 constexpr size_t GRID_TAIL = 32768;            // bytes: header + GRID_PARTS * 7 partials
 constexpr int GRID_MODE_CELLS = 0, GRID_MODE_FALLBACK = 1;
 
-// The workgroups (and partials) of the scans for n voxels: one per 256 voxels, 64 at least. Each
-// workgroup reads every partial, so a small set's scans are short only with few of them (table and
-// plan of 15 K voxels 56.6 -> 52.7 us, of 1.5 K 52 -> 47, against 1024 always).
+// The workgroups (and partials) of a scan over n voxels: one per 256 voxels, 64 at least. Each
+// workgroup reads every partial, so a small set's scans are short only with few of them.
 inline int grid_parts(int64_t n) {
     const int64_t p = ((n + 255) / 256 + 63) / 64 * 64;
     return (int)(p < 64 ? 64 : p > GRID_PARTS ? GRID_PARTS : p);
+}
+// The passes over the directory and over the blocks, whose sizes follow the bounding box and are
+// known on the device only, are launched with 256 workgroups at least, the first dir_parts (walk_parts)
+// of which have work and partials: DIR_WORDS directory words a workgroup and round, a block a wave.
+// Ordered plans, us so, with workgroups by the voxels alone (64 here) of a word a thread, and with 1024
+// always: 2 K voxels spread over 1000^3 (a directory of 2^21 words, 2.5 K blocks) 92, 160 and 92; over
+// 500^3 91, 107 and 92; 14.5 K of a shell 52, 52 and 55.
+constexpr int DIR_WORDS = 1024;
+inline int grid_workgroups(int64_t n) {
+    const int np = grid_parts(n);
+    return np < 256 ? 256 : np;
+}
+__device__ __forceinline__ int dir_parts(int64_t dir_n, int workgroups) {
+    return (int)min<int64_t>(workgroups, (dir_n + DIR_WORDS - 1) / DIR_WORDS);
+}
+__device__ __forceinline__ int walk_parts(int nblocks, int voxel_parts, int workgroups) {
+    return max(voxel_parts, min(workgroups, (nblocks + 3) / 4));
+}
+// words of one of them, a multiple of DIR_WORDS
+__device__ __forceinline__ int64_t dir_chunk(int64_t dir_n, int parts) {
+    return ((dir_n + parts - 1) / parts + DIR_WORDS - 1) / DIR_WORDS * DIR_WORDS;
 }
 
 struct GridHdr {

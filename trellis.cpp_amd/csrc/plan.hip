@@ -53,10 +53,12 @@ __device__ __forceinline__ uint64_t pack_xyz(int32_t x, int32_t y, int32_t z) {
 __global__ __launch_bounds__(WK_NT) void k_walk_count(const int32_t* __restrict__ coords, int64_t n,
                                                       const int32_t* __restrict__ dir, const GridHdr* __restrict__ hdr,
                                                       int32_t* __restrict__ counts, uint8_t* __restrict__ pres,
-                                                      int32_t* __restrict__ parts, int np) {
+                                                      int32_t* __restrict__ parts, int voxel_parts) {
     __shared__ int sW[WK_NT / 64];
     __shared__ int sB[WK_NT / 64];
     if (hdr->mode != GRID_MODE_CELLS) return;
+    const int np = walk_parts(hdr->nblocks, voxel_parts, gridDim.x);
+    if ((int)blockIdx.x >= np) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const GridRef g = grid_ref(dir, hdr);
     const int64_t nb = hdr->nblocks, bchunk = (nb + np - 1) / np;
@@ -90,7 +92,7 @@ __global__ __launch_bounds__(WK_NT) void k_walk_count(const int32_t* __restrict_
 // The stores of the walk: the row (order) and packed coordinates (wc) of every voxel -- block
 // voxels from their block's start, column by column, then the left-out voxels after all block
 // voxels. Every workgroup sums the partials before it (and all block partials) itself.
-// Workgroups from np on carry the neighbour-table probe (pj), when asked for: the walk is
+// Workgroups from nw on carry the neighbour-table probe (pj), when asked for: the walk is
 // latency-bound and the probe bound by its table stores, so the two share the launch (2-3 % off
 // the table + plan call, against the probe as a launch of its own; a third of the probe on the
 // count launch instead measured the same).
@@ -100,17 +102,19 @@ __global__ __launch_bounds__(WK_NT) void k_walk_emit(const int32_t* __restrict__
                                                      const int32_t* __restrict__ cell_of,
                                                      const int32_t* __restrict__ parts, int32_t* __restrict__ order,
                                                      uint64_t* __restrict__ wc, int32_t* __restrict__ list_n,
-                                                     ProbeJob pj, int np) {
+                                                     ProbeJob pj, int voxel_parts, int nw) {
     __shared__ int sW[WK_NT / 64];
     __shared__ int sS[3][WK_NT / 64];
     __shared__ int sStart[WK_NT];
-    if ((int)blockIdx.x >= np) {
-        const int64_t i = pj.v0 + (int64_t)(blockIdx.x - np) * WK_NT + threadIdx.x;
+    if ((int)blockIdx.x >= nw) {
+        const int64_t i = pj.v0 + (int64_t)(blockIdx.x - nw) * WK_NT + threadIdx.x;
         if (i < pj.v1) probe_voxel(coords, n, i, dir, hdr, pj.hash, pj.nbr);
         return;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) *list_n = 0;   // the plan kernels' list of table tiles
     if (hdr->mode != GRID_MODE_CELLS) return;
+    const int np = walk_parts(hdr->nblocks, voxel_parts, nw);
+    if ((int)blockIdx.x >= np) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const GridRef g = grid_ref(dir, hdr);
     const int64_t nb = hdr->nblocks, bchunk = (nb + np - 1) / np;
@@ -906,19 +910,19 @@ static int plan_on_grid(const int32_t* nbr, const int32_t* coords, int64_t n, vo
     const PlanView pv = carve_plan(plan, n_tiles);
     // the table probe, when asked for, rides on the walk's emit launch
     ProbeJob pj;
-    const int np = grid_parts(n);
-    int64_t ge = np;
+    const int np = grid_parts(n), nw = grid_workgroups(n);
+    int64_t ge = nw;
     if (probe && probe->nbr) {
         pj = *probe;
         pj.v0 = 0;
         pj.v1 = n;
         ge += ceil_div(n, WK_NT);
     }
-    hipLaunchKernelGGL(k_walk_count, dim3((unsigned)np), dim3(WK_NT), 0, s, coords, n, dir, gt.hdr, ps.counts,
+    hipLaunchKernelGGL(k_walk_count, dim3((unsigned)nw), dim3(WK_NT), 0, s, coords, n, dir, gt.hdr, ps.counts,
                        ps.pres, gt.parts, np);
     TSP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_walk_emit, dim3((unsigned)ge), dim3(WK_NT), 0, s, coords, n, dir, gt.hdr, ps.counts,
-                       ps.pres, ps.cell_of, gt.parts, ps.order, ps.wc, list_n, pj, np);
+                       ps.pres, ps.cell_of, gt.parts, ps.order, ps.wc, list_n, pj, np, nw);
     TSP_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_plan_window, dim3((unsigned)n_tiles), dim3(HB_PLAN_NT), 0, s, n, ps.order, ps.wc, dir,
                        ps.pres, gt.hdr, pv, list, list_n);
