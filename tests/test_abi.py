@@ -380,3 +380,24 @@ def test_convnext_mlp_validation(pkg):
     assert mlp(xn=ctypes.c_void_p(0x1008)) == 1 and "aligned" in _err(pkg)
     assert mlp(out=FAKE) == 1 and "alias" in _err(pkg)
     assert mlp(n=0, packed=NULL) == 0
+
+
+def test_library_gemm_needs_no_workspace(pkg):
+    """The linear layers call the GEMM library without a workspace: of the heuristic's results only one
+    whose state is success and that asks for none may run."""
+    class Result(ctypes.Structure):   # hipblasLtMatmulHeuristicResult_t
+        _fields_ = [("algo", ctypes.c_uint8 * 24), ("workspace", ctypes.c_size_t), ("state", ctypes.c_int),
+                    ("waves", ctypes.c_float), ("reserved", ctypes.c_int * 4)]
+    usable = pkg.lib()["_ZN3tsp13blaslt_usableEPK33_hipblasLtMatmulHeuristicResult_ti"]
+    usable.restype = ctypes.c_int
+
+    def pick(*results):
+        a = (Result * max(1, len(results)))()
+        for k, (ws, state) in enumerate(results):
+            a[k].workspace, a[k].state = ws, state
+        return usable(a, len(results))
+    assert pick() == -1
+    assert pick((0, 0), (0, 0)) == 0
+    assert pick((4096, 0), (0, 0)) == 1
+    assert pick((0, 7), (4096, 0), (0, 0)) == 2
+    assert pick((4096, 0), (0, 3)) == -1

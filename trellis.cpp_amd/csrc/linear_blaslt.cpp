@@ -57,6 +57,15 @@ struct Gemm {
 
 }  // namespace
 
+// The first of the heuristic's results that may run without a workspace, -1 when there is none: a
+// result's other fields hold only with state SUCCESS, and its kernel writes partial sums to the
+// workspace it asks for.
+int blaslt_usable(const hipblasLtMatmulHeuristicResult_t* results, int count) {
+    for (int k = 0; k < count; ++k)
+        if (results[k].state == HIPBLAS_STATUS_SUCCESS && results[k].workspaceSize == 0) return k;
+    return -1;
+}
+
 bool blaslt_eligible(int x_dtype, int weight_dtype, int out_dtype, int ci, int co, const void* x,
                      const void* w, const void* out) {
     if (x_dtype == TSP_F32 || x_dtype != weight_dtype) return false;
@@ -135,14 +144,14 @@ static int blaslt_linear_rows(const void* x, int xdt, int64_t n, int ci, const v
         AlgoEntry e;
         hipblasLtMatmulPreference_t pref = nullptr;
         uint64_t ws = 0;
-        hipblasLtMatmulHeuristicResult_t res{};
-        int count = 0;
+        hipblasLtMatmulHeuristicResult_t res[4]{};
+        int count = 0, pick = -1;
         if (hipblasLtMatmulPreferenceCreate(&pref) == HIPBLAS_STATUS_SUCCESS &&
             hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws)) == HIPBLAS_STATUS_SUCCESS &&
-            hipblasLtMatmulAlgoGetHeuristic(h, g.desc, g.a, g.b, g.c, g.d, pref, 1, &res, &count) == HIPBLAS_STATUS_SUCCESS &&
-            count > 0) {
+            hipblasLtMatmulAlgoGetHeuristic(h, g.desc, g.a, g.b, g.c, g.d, pref, 4, res, &count) == HIPBLAS_STATUS_SUCCESS &&
+            (pick = blaslt_usable(res, std::min(count, 4))) >= 0) {
             e.ok = true;
-            e.algo = res.algo;
+            e.algo = res[pick].algo;
         }
         if (pref) hipblasLtMatmulPreferenceDestroy(pref);
         it = g_algos.emplace(key, e).first;
