@@ -382,6 +382,22 @@ def test_convnext_mlp_validation(pkg):
     assert mlp(n=0, packed=NULL) == 0
 
 
+@pytest.mark.parametrize("call", [
+    lambda p, t: p.mask_positive(t.zeros((4, 8), dtype=t.float16)),
+    lambda p, t: p.mask_positive(t.zeros((4, 8), dtype=t.bfloat16)),
+    lambda p, t: p.linear(t.zeros((4, 32)), t.zeros((8, 32)), t.zeros(8, dtype=t.float16)),
+    lambda p, t: p.linear(t.zeros((4, 32)), t.zeros((8, 32)), t.zeros(7)),
+    lambda p, t: p.linear_ex(t.zeros((4, 32)), t.zeros((8, 32)), t.zeros(8, dtype=t.bfloat16)),
+    lambda p, t: p.layer_norm(t.zeros((4, 32)), t.zeros(32, dtype=t.float16), t.zeros(32)),
+    lambda p, t: p.layer_norm(t.zeros((4, 32)), t.zeros(32), t.zeros(31))])
+def test_float32_vectors(pkg, call):
+    """The kernels read these operands as float32 through their pointers: a 16-bit or shorter one, read
+    past its end, is refused before any device work."""
+    import torch
+    with pytest.raises(ValueError, match="float32"):
+        call(pkg, torch)
+
+
 def test_library_gemm_needs_no_workspace(pkg):
     """The linear layers call the GEMM library without a workspace: of the heuristic's results only one
     whose state is success and that asks for none may run."""

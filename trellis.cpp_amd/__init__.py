@@ -332,6 +332,15 @@ def _check_out(out, n: int, co: int, dtype, device):
         raise ValueError(f"out must live on {device}, got {out.device}")
 
 
+def _f32_vec(t, n: int, name: str):
+    """An optional float32 vector of at least n elements: the kernels read n through its pointer."""
+    if t is None:
+        return None
+    if t.dtype != _torch().float32 or t.numel() < n:
+        raise ValueError(f"{name} must be float32 with {n} elements")
+    return t.contiguous()
+
+
 def _check_nbr(nbr, n: int, device):
     torch = _torch()
     if nbr.dtype != torch.int32 or nbr.numel() != 27 * n or not nbr.is_contiguous():
@@ -570,6 +579,7 @@ def subdivide(mask, coords, stream=None):
 def linear(x, weight, bias=None, out_dtype=None, stream=None):
     """x [N,Ci] . W^T + bias for W [Co,Ci] -> [N,Co] (fp32 accumulation)."""
     torch = _torch()
+    bias = _f32_vec(bias, weight.shape[0], "bias")
     _require_cuda(x, weight, bias)
     n, ci = x.shape
     co = weight.shape[0]
@@ -591,6 +601,7 @@ def linear_ex(x, weight, bias=None, act: str = "none", residual=None, out_dtype=
     bias, activation and residual in its epilogue (16-bit x and W of one dtype; raises
     TspError UNSUPPORTED otherwise)."""
     torch = _torch()
+    bias = _f32_vec(bias, weight.shape[0], "bias")
     _require_cuda(x, weight, bias, residual)
     n, ci = x.shape
     co = weight.shape[0]
@@ -612,6 +623,7 @@ def layer_norm(x, gamma=None, beta=None, eps: float = 1e-6, silu: bool = False, 
                stream=None):
     """Row LayerNorm over channels (biased variance) [* gamma + beta] [then SiLU]."""
     torch = _torch()
+    gamma, beta = _f32_vec(gamma, x.shape[1], "gamma"), _f32_vec(beta, x.shape[1], "beta")
     _require_cuda(x, gamma, beta)
     xc = x.contiguous()
     n, c = xc.shape
@@ -650,6 +662,8 @@ def c2s_skip_add(x, gidx, acc, stream=None):
 def mask_positive(logits, stream=None):
     """uint8 mask of logits > 0 (float32 input, any shape)."""
     torch = _torch()
+    if logits.dtype != torch.float32:   # (the kernel would read twice a 16-bit tensor's bytes)
+        raise ValueError(f"logits must be float32, got {logits.dtype}")
     _require_cuda(logits)
     lc = logits.contiguous()
     mask = torch.empty(lc.shape, dtype=torch.uint8, device=lc.device)
