@@ -122,7 +122,7 @@ def _front_us(tsp, b, ws, ws_bytes):
     return best
 
 
-@pytest.mark.parametrize("n,cin,cout", [(24001, 256, 128), (12001, 512, 256), (9001, 256, 384)])
+@pytest.mark.parametrize("n,cin,cout", [(24001, 256, 128), (30001, 256, 128), (14001, 256, 128), (12001, 512, 256), (9001, 256, 384)])
 @pytest.mark.parametrize("keep", list(MASKS))
 def test_uneven_octants(gpu_lib, shells, n, cin, cout, keep):
     """Each octant's tiles are its own (none is empty or reads its rows from memory), a plan that does
@@ -146,7 +146,10 @@ def test_uneven_octants(gpu_lib, shells, n, cin, cout, keep):
         assert direct == 0 and (rows <= 512).all()
         if fits:
             assert most <= -(-n // 512)
-        assert bool(fits) == (keep in ("half", "rare", "two rates", "none")) or cout == 384
+        if keep in ("one full", "half full") or (n == 14001 and keep != "rare"):   # (14 K: a round on either plan)
+            assert not fits
+        elif keep in ("half", "rare") and n != 14001:
+            assert fits
     st, want = _run(gpu_lib, b, ws, less)
     assert st == 0 and torch.equal(got, want)
     assert _front_us(gpu_lib, b, ws, full) < 2 * _front_us(gpu_lib, b, ws, less) + 50

@@ -125,9 +125,9 @@ struct OctantScatter {
 // 1100 us).
 struct OctantPlan {
     int cap = 0;          // tiles, at most
-    // The conv's time in rounds of units, in tenths: on the parents' plan base_cost, on the octant plan
-    // 10 ceil(ceil(T mul / 8) / fit) for T tiles of the octant that has most (by_sum: of all octants).
-    int base_cost = 0, mul = 0, fit = 0;
+    // conv1's time in hundredths of a round of units: base_cost on the parents' plan; on the octant plan
+    // octant_cost of the tiles of the octant that has most (by_sum: of all octants), and build_cost.
+    int base_cost = 0, build_cost = 0, mul = 0, fit = 0;
     bool by_sum = false;
     size_t plan_bytes = 0, member_bytes = 0, count_bytes = 0;
 };

@@ -716,15 +716,23 @@ __global__ __launch_bounds__(HB_M) void k_octant_count(const int32_t* __restrict
 // kept by 35 %).
 constexpr int OCT_SPAN = 1152;
 
+// Hundredths of a round that the units of `tiles` tiles take: a round of them has a fixed part, and
+// the units of a round run faster the fewer they are (14 K 256 -> 128 and 8 K 512 -> 256, whose octant
+// plan has 0.47 and 0.53 of a round for 0.88 and 1: 47 and 110 us off a round's 149 and 300).
+__host__ __device__ inline int64_t octant_cost(const OctantPlan& op, int64_t tiles) {
+    const int64_t units = (tiles * op.mul + 7) / 8;
+    return 30 * ((units + op.fit - 1) / op.fit) + 70 * units / op.fit;
+}
+
 // One workgroup, 128 threads an octant: the counts' exclusive prefixes over the tiles, in place; then
-// each octant's tiles, and whether the plan is taken: where its tiles fit the space and its rounds of
-// units are a tenth fewer than the parents' plan's. A unit costs about the same on either, however
-// many of its MFMAs are skipped, and a workgroup of the large-grid kernel keeps its octant, so the
-// fullest octant decides there. 60 K 256 -> 128, us up to conv2 on the octant plan and on the parents':
-// every octant kept by 27 % 360 and 708, by 75 % 631 and 706; one octant by all and seven by 5 % (not
-// taken, some 15 us for the build's launches) 741 and 671 -- with the mean's tiles for every octant it
-// took 4085. A tile whose rows are read from memory runs eight times as long, on either plan: seven
-// rounds more for its workgroup.
+// each octant's tiles, and whether the plan is taken: where its tiles fit the space and its units and
+// its build take a tenth less time than the units of the parents' plan. A unit costs about the same
+// on either, however many of its MFMAs are skipped, and a workgroup of the large-grid kernel keeps its
+// octant, so the fullest octant decides there. 60 K 256 -> 128, us up to conv2 on the octant plan and
+// on the parents': every octant kept by 27 % 360 and 708, by 75 % 631 and 706; one octant by all and
+// seven by 5 % (not taken, some 15 us for the build's launches) 741 and 671 -- with the mean's tiles
+// for every octant it took 4085. A tile whose rows are read from memory runs eight times as long, on
+// either plan: seven rounds more for its workgroup.
 __global__ __launch_bounds__(1024) void k_octant_scan(int64_t n, int64_t n_tiles, const int32_t* __restrict__ hdr,
                                                       OctantPlan op, int32_t* __restrict__ counts,
                                                       OctantTiles* __restrict__ oct) {
@@ -768,11 +776,10 @@ __global__ __launch_bounds__(1024) void k_octant_scan(int64_t n, int64_t n_tiles
             total += sO.tiles[k];
             most = max(most, sO.tiles[k]);
         }
-        const int64_t units = ((op.by_sum ? total : most) * (int64_t)op.mul + 7) / 8;
-        const int64_t cost = 10 * ((units + op.fit - 1) / op.fit), base = op.base_cost + (sD ? 70 : 0);
+        const int64_t cost = octant_cost(op, op.by_sum ? total : most) + op.build_cost, base = op.base_cost + (sD ? 700 : 0);
         // (the launch's grid is the parents' tiles')
-        sO.fits = total <= op.cap && total <= 8 * n_tiles && most <= n_tiles && 10 * cost <= 9 * base;
-        sO.spare = base - cost >= 160 ? total / 128 : base - cost >= 80 ? 1 : 0;
+        sO.fits = total <= op.cap && total <= 8 * n_tiles && most <= n_tiles && 11 * cost <= 10 * base;
+        sO.spare = base - cost >= 1600 ? total / 128 : base - cost >= 800 ? 1 : 0;
         sO.direct = 0;
         sO.total = total;
         sO.most = most;
@@ -847,17 +854,21 @@ bool octant_plan_spec(int64_t n, int64_t m, int cin, int cout, OctantPlan& op) {
     const int64_t cap = 11 * ceil_div(m, rows) / 10 + 16, tiles = ceil_div(n, HB_M);
     if (cap > INT32_MAX / 16) return false;
     op.cap = (int)cap;
+    const int nkc = cin / HB_KC;
     if (rgw) {   // the units of all octants' tiles, any compute unit
         op.by_sum = true;
         op.mul = cout / (64 * ncg) * (4 / rgw);
         op.fit = std::max(1, cus / 8);
-        op.base_cost = (int)(10 * ceil_div(ceil_div(8 * tiles * op.mul, 8), op.fit));
+        op.base_cost = (int)octant_cost(op, 8 * tiles);
+        op.build_cost = (int)(5000 / (6 + (rgw * ncg == 4 ? 4.6 : rgw * ncg == 2 ? 2.45 : 1.6) * nkc));
     } else {     // a workgroup keeps its column, so its octant
         op.by_sum = false;
         op.mul = co / 128;
         op.fit = std::max(1, cus / 8 / op.mul) * op.mul;
-        const int64_t split = cout == 128 ? 0 : column_split_tiles(tiles, op.mul, cus);   // (a thin last round: 0.65)
-        op.base_cost = (int)(10 * ceil_div(ceil_div((split ? split : tiles) * op.mul, 8), op.fit) + (split ? 6 : 0));
+        op.base_cost = (int)octant_cost(op, tiles);
+        const int64_t split = cout == 128 ? 0 : column_split_tiles(tiles, op.mul, cus);   // (a thin last round: 0.6)
+        if (split) op.base_cost = std::min(op.base_cost, (int)octant_cost(op, split) + 60);
+        op.build_cost = (int)(5500 / (9.3 * nkc));
     }
     op.plan_bytes = plan_tile_bytes(cap);
     op.member_bytes = (size_t)cap * HB_M * 4;
