@@ -1,5 +1,6 @@
 """The C2S block's octant plan (csrc/plan.hip) where it is not the usual call: a workspace without
-room for it; masks that keep some octants far more often than others."""
+room for it; masks that keep some octants far more often than others; the
+block in parts; weights and a row 0 that are not finite."""
 from __future__ import annotations
 
 import ctypes
@@ -153,3 +154,65 @@ def test_uneven_octants(gpu_lib, shells, n, cin, cout, keep):
     st, want = _run(gpu_lib, b, ws, less)
     assert st == 0 and torch.equal(got, want)
     assert _front_us(gpu_lib, b, ws, full) < 2 * _front_us(gpu_lib, b, ws, less) + 50
+
+
+def _part(tsp, b, ws, ws_bytes, out, part, t0=0, nt=-1):
+    import torch
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    return tsp.lib().tsp_c2s_part(ptr(b["x"]), b["n"], b["cin"], ptr(b["nbr"]), ptr(b["plan"]), ptr(b["mask"]),
+                                  ptr(b["mstart"]), ptr(b["gidx"]), b["m"], b["cout"], ptr(b["cnbr"]), ptr(b["cplan"]),
+                                  ctypes.byref(_weights(tsp, b["p"])), ptr(out), None, 2, ptr(ws), ws_bytes, 0, part, t0, nt,
+                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+
+@pytest.mark.parametrize("n,cin,cout", [(24001, 256, 128), (12001, 512, 256)])
+def test_parts(gpu_lib, shells, n, cin, cout):
+    """The front part once, then conv2 over ranges of the child plan's tiles, and all parts at once on
+    a stream of its own: the same bits, and nothing outside the range is written."""
+    import torch
+    print(f"[octant plan] parts n={n} {cin}->{cout}", flush=True)
+    b = _block(gpu_lib, shells, n, cin, cout, [0.5] * 8, key="f16")
+    full = _bytes(gpu_lib, b)
+    ws = torch.empty(full, dtype=torch.uint8, device="cuda")
+    st, want = _run(gpu_lib, b, ws, full)
+    assert st == 0
+    ws.fill_(0xA5)
+    out = torch.full((b["m"], cout), float("nan"), device="cuda")
+    tiles = -(-b["m"] // 512)
+    assert _part(gpu_lib, b, ws, full, out, 1) == 0 and bool(out.isnan().all())
+    cuts = [0, 1, tiles // 3, tiles - 1, tiles]
+    for t0, t1 in zip(cuts[:-1], cuts[1:]):
+        assert _part(gpu_lib, b, ws, full, out, 2, t0, t1 - t0) == 0
+        torch.cuda.synchronize()
+        assert int((~out[:, 0].isnan()).sum()) == min(b["m"], 512 * t1)
+    assert torch.equal(out, want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        st, got = _run(gpu_lib, b, ws, full)
+    torch.cuda.current_stream().wait_stream(side)
+    assert st == 0 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("bad", ["weight inf", "weight nan", "row 0 nan"])
+@pytest.mark.parametrize("n,cin,cout", [(24001, 256, 128), (30001, 256, 128), (12001, 512, 256)])
+def test_values_not_finite(gpu_lib, shells, n, cin, cout, bad):
+    """On the octant plan and on the parents' plan (whose conv is tested against the other kernels): the
+    same values where they are numbers, NaN in the same places."""
+    import torch
+    print(f"[octant plan] {bad} n={n} {cin}->{cout}", flush=True)
+    b = _block(gpu_lib, shells, n, cin, cout, [0.5] * 8)
+    value = float("inf") if bad.endswith("inf") else float("nan")
+    if bad.startswith("weight"):
+        b["p"]["conv1.weight"][3 * cout + 7, 4, 11] = value   # (an octant's channel)
+        b["p"]["conv1.packed"] = gpu_lib.conv_weight_pack(b["p"]["conv1.weight"])
+    else:
+        b["x"][0, 5] = value
+    full, less = _bytes(gpu_lib, b), _without_plan(n, b["m"], cin, cout)
+    assert less < full
+    ws = torch.empty(full, dtype=torch.uint8, device="cuda")
+    (st, got), (st2, want) = _run(gpu_lib, b, ws, full), _run(gpu_lib, b, ws, less)
+    assert st == 0 and st2 == 0
+    assert bool(want.isnan().any()) and torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(0.0), want.nan_to_num(0.0))
+
