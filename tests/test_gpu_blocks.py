@@ -78,6 +78,34 @@ def test_linear_ex(gpu_lib, orc, n, ci, co):
         gpu_lib.linear_ex(_t(np.ones((4, 32), np.float32)), _t(np.ones((64, 32), np.float32)))
 
 
+@pytest.mark.parametrize("n,ci,co,act,residual", [(8200, 512, 2048, "silu", False), (16400, 512, 2048, "silu", False),
+                                                  (20000, 256, 1024, "silu", False), (35001, 512, 2048, "silu", False),
+                                                  (70000, 256, 1024, "silu", False), (70000, 4096, 1024, "none", True),
+                                                  (134000, 256, 64, "none", True), (134000, 512, 8, "none", False)])
+@pytest.mark.parametrize("key", ["bfloat16", "float16"])
+def test_linear_ex_without_workspace(gpu_lib, n, ci, co, act, residual, key):
+    """Shapes for which a build of the GEMM library lists first a kernel that needs a workspace, or (70 K of
+    4096 -> 1024) none that does not: sampled rows, of both halves, against fp64."""
+    import torch
+    print(f"[linear] no workspace n={n} {ci}->{co} {act} residual={residual} {key}", flush=True)
+    dt = getattr(torch, key)
+    g = torch.Generator(device="cuda").manual_seed(n + co)
+    x = torch.randn((n, ci), generator=g, device="cuda").to(dt)
+    w = (torch.randn((co, ci), generator=g, device="cuda") * ci ** -0.5).to(dt)
+    b = torch.randn(co, generator=g, device="cuda")
+    r = torch.randn((n, co), generator=g, device="cuda") if residual else None
+    out = gpu_lib.linear_ex(x, w, b, act=act, residual=r, out_dtype=torch.float32 if act == "none" else dt)
+    rows = torch.cat([torch.arange(300), torch.arange(n // 2 - 300, n // 2 + 300), torch.arange(n - 300, n)]).cuda()
+    ref = x[rows].cpu().double() @ w.cpu().double().t() + b.cpu().double()
+    if act == "silu":
+        ref = ref / (1 + torch.exp(-ref))
+    if residual:
+        ref = ref + r[rows].cpu().double()
+    # f32 sums; one rounding of the result to 16 bits
+    tol = 1e-5 if act == "none" else 2.0 ** (-8 if key == "bfloat16" else -11)
+    assert float((out[rows].cpu().double() - ref).abs().max() / ref.abs().max()) < tol
+
+
 def test_linear_ex_chunked_over_2gib(gpu_lib, orc):
     """tsp_linear_ex where one operand spans more than 2 GiB: the decoder's last-stage ConvNeXt
     hidden layer, 2,445,586 rows x (128 -> 512) bf16 with f32 output (5.0 GB), which the library

@@ -4,7 +4,11 @@
 // column-major product D (co x n) = op(W') (co x ci) . x' (ci x n) with W' = W viewed column-major
 // (ci x co, transposed by the op) and x' = x viewed column-major. Bias and SiLU run in the GEMM's
 // epilogue (fp32, before the output's rounding); the residual enters as C with beta = 1.
-// Algorithms come from hipBLASLt's heuristic with no workspace, cached per shape and device.
+// Algorithms come from hipBLASLt's heuristic with no workspace, cached per shape and device. Some builds
+// of the library return kernels that need one all the same (stream-K kernels, whose partial sums then
+// go to a null pointer: illegal accesses at 8.2 K rows of 512 -> 2048, 70 K of 256 -> 1024, while 35 K
+// of 512 -> 2048 ran), so only results that ask for none are used, and where there is none among
+// them, the call is cut into fewer rows.
 #include <hipblaslt/hipblaslt.h>
 
 #include <map>
@@ -76,7 +80,8 @@ bool blaslt_eligible(int x_dtype, int weight_dtype, int out_dtype, int ci, int c
 }
 
 static int blaslt_linear_rows(const void* x, int xdt, int64_t n, int ci, const void* w, const float* bias,
-                              int co, int act, const float* residual, void* out, int odt, hipStream_t s);
+                              int co, int act, const float* residual, void* out, int odt, hipStream_t s,
+                              bool launch);
 
 // Rows of one library call: no operand (x, out, residual) of a call spans 2^31 bytes or more (a
 // multiple of 256 rows where one fits; 0 when not even one row does).
@@ -89,23 +94,40 @@ int64_t blaslt_rows_per_call(int ci, int co, int xdt, int odt, bool residual) {
 }
 
 // Row chunks of blaslt_rows_per_call rows: one library call never addresses 2^31 bytes or more
-// in an operand (the composite blocks already bound their hidden layers to 1 GiB).
+// in an operand (the composite blocks already bound their hidden layers to 1 GiB). Chunks for which the
+// library has no usable algorithm are halved down to 4096 rows; nothing is launched before every
+// chunk has one.
 int blaslt_linear(const void* x, int xdt, int64_t n, int ci, const void* w, const float* bias,
                   int co, int act, const float* residual, void* out, int odt, hipStream_t s) {
-    const int64_t rows = blaslt_rows_per_call(ci, co, xdt, odt, residual != nullptr);
+    if (n <= 0) return TSP_OK;
+    int64_t rows = std::min(n, blaslt_rows_per_call(ci, co, xdt, odt, residual != nullptr));
     TSP_REQUIRE(rows > 0, TSP_ERR_UNSUPPORTED, "linear: a row of ci=%d co=%d spans 2 GiB", ci, co);
-    for (int64_t r0 = 0; r0 < n; r0 += rows) {
-        const int64_t nr = std::min(rows, n - r0);
-        const int st = blaslt_linear_rows(static_cast<const char*>(x) + r0 * ci * (int64_t)dtype_size(xdt), xdt, nr,
-                                          ci, w, bias, co, act, residual ? residual + r0 * co : nullptr,
-                                          static_cast<char*>(out) + r0 * co * (int64_t)dtype_size(odt), odt, s);
-        if (st != TSP_OK) return st;
+    auto each = [&](bool launch) {
+        for (int64_t r0 = 0; r0 < n; r0 += rows) {
+            const int64_t nr = std::min(rows, n - r0);
+            const int st = blaslt_linear_rows(static_cast<const char*>(x) + r0 * ci * (int64_t)dtype_size(xdt), xdt, nr,
+                                              ci, w, bias, co, act, residual ? residual + r0 * co : nullptr,
+                                              static_cast<char*>(out) + r0 * co * (int64_t)dtype_size(odt), odt, s, launch);
+            if (st != TSP_OK) return st;
+            if (!launch && r0 == 0 && n % rows && n > 2 * rows) r0 = n / rows * rows - rows;   // (then the last, shorter one)
+        }
+        return (int)TSP_OK;
+    };
+    for (;;) {
+        const bool one = rows >= n;
+        const int st = each(one);
+        if (st == TSP_OK) {
+            clear_error();
+            return one ? st : each(true);
+        }
+        if (st != TSP_ERR_UNSUPPORTED || rows <= 4096) return st;
+        rows = ceil_div(rows, 512) * 256;
     }
-    return TSP_OK;
 }
 
 static int blaslt_linear_rows(const void* x, int xdt, int64_t n, int ci, const void* w, const float* bias,
-                              int co, int act, const float* residual, void* out, int odt, hipStream_t s) {
+                              int co, int act, const float* residual, void* out, int odt, hipStream_t s,
+                              bool launch) {
     int dev = 0;
     TSP_CHECK_HIP(hipGetDevice(&dev));
     TSP_REQUIRE(dev >= 0 && dev < kMaxDevices, TSP_ERR_INVALID, "linear: device %d out of range", dev);
@@ -144,12 +166,18 @@ static int blaslt_linear_rows(const void* x, int xdt, int64_t n, int ci, const v
         AlgoEntry e;
         hipblasLtMatmulPreference_t pref = nullptr;
         uint64_t ws = 0;
-        hipblasLtMatmulHeuristicResult_t res[4]{};
+        // the heuristic's first choice, or the first that is usable of many
+        hipblasLtMatmulHeuristicResult_t res[64]{};
         int count = 0, pick = -1;
         if (hipblasLtMatmulPreferenceCreate(&pref) == HIPBLAS_STATUS_SUCCESS &&
-            hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws)) == HIPBLAS_STATUS_SUCCESS &&
-            hipblasLtMatmulAlgoGetHeuristic(h, g.desc, g.a, g.b, g.c, g.d, pref, 4, res, &count) == HIPBLAS_STATUS_SUCCESS &&
-            (pick = blaslt_usable(res, std::min(count, 4))) >= 0) {
+            hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws)) == HIPBLAS_STATUS_SUCCESS) {
+            for (int want : {1, 64}) {
+                if (hipblasLtMatmulAlgoGetHeuristic(h, g.desc, g.a, g.b, g.c, g.d, pref, want, res, &count) == HIPBLAS_STATUS_SUCCESS)
+                    pick = blaslt_usable(res, std::min(count, want));
+                if (pick >= 0) break;
+            }
+        }
+        if (pick >= 0) {
             e.ok = true;
             e.algo = res[pick].algo;
         }
@@ -160,6 +188,7 @@ static int blaslt_linear_rows(const void* x, int xdt, int64_t n, int ci, const v
         set_error("linear: hipBLASLt has no algorithm for n=%lld ci=%d co=%d", (long long)n, ci, co);
         return TSP_ERR_UNSUPPORTED;
     }
+    if (!launch) return TSP_OK;
     const float alpha = 1.f, beta = residual ? 1.f : 0.f;
     const hipblasStatus_t st = hipblasLtMatmul(h, g.desc, &alpha, w, g.a, x, g.b, &beta,
                                                residual ? static_cast<const void*>(residual) : out, g.c,

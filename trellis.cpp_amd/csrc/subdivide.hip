@@ -15,9 +15,7 @@
 namespace tsp {
 namespace {
 
-constexpr int SD_THREADS = 1024;
-constexpr int SD_PER_THREAD = 1;
-constexpr int SD_ITEMS = SD_THREADS * SD_PER_THREAD;   // parents per block
+constexpr int SD_THREADS = 1024;   // a thread a parent
 
 __device__ __forceinline__ uint32_t octant_bits(const uint8_t* __restrict__ mask, int64_t i) {
     uint32_t m = 0;
@@ -51,13 +49,9 @@ __device__ __forceinline__ int32_t block_exclusive_scan(int32_t v, int32_t* tota
 
 __global__ __launch_bounds__(SD_THREADS) void k_block_counts(const uint8_t* __restrict__ mask,
                                                             int64_t n, int32_t* block_sums) {
-    const int64_t p0 = (int64_t)blockIdx.x * SD_ITEMS + (int64_t)threadIdx.x * SD_PER_THREAD;
-    int32_t c = 0;
-#pragma unroll
-    for (int k = 0; k < SD_PER_THREAD; ++k)
-        if (p0 + k < n) c += __popc(octant_bits(mask, p0 + k));
+    const int64_t i = (int64_t)blockIdx.x * SD_THREADS + threadIdx.x;
     int32_t tot;
-    block_exclusive_scan(c, &tot);
+    block_exclusive_scan(i < n ? __popc(octant_bits(mask, i)) : 0, &tot);
     if (threadIdx.x == 0) block_sums[blockIdx.x] = tot;
 }
 
@@ -87,31 +81,19 @@ __global__ __launch_bounds__(SD_THREADS) void k_emit_children(
     const uint8_t* __restrict__ mask, const int32_t* __restrict__ coords, int64_t n,
     const int32_t* __restrict__ block_offsets, int32_t* __restrict__ mstart,
     int32_t* __restrict__ child, int32_t* __restrict__ gidx) {
-    __shared__ int32_t sC[3 * SD_ITEMS];          // the block's parents
-    __shared__ uint16_t sList[8 * SD_ITEMS];      // octant + 8 parent of each child
-    const int64_t b0 = (int64_t)blockIdx.x * SD_ITEMS;
-    const int tid = threadIdx.x, items = (int)min<int64_t>(SD_ITEMS, n - b0);
+    __shared__ int32_t sC[3 * SD_THREADS];          // the block's parents
+    __shared__ uint16_t sList[8 * SD_THREADS];      // octant + 8 parent of each child
+    const int64_t b0 = (int64_t)blockIdx.x * SD_THREADS;
+    const int tid = threadIdx.x, items = (int)min<int64_t>(SD_THREADS, n - b0);
     for (int k = tid; k < 3 * items; k += SD_THREADS) sC[k] = coords[3 * b0 + k];
-    const int l0 = tid * SD_PER_THREAD;
-    uint32_t bits[SD_PER_THREAD];
-    int32_t c = 0;
-#pragma unroll
-    for (int k = 0; k < SD_PER_THREAD; ++k) {
-        bits[k] = (l0 + k < items) ? octant_bits(mask, b0 + l0 + k) : 0u;
-        c += __popc(bits[k]);
-    }
+    uint32_t b = tid < items ? octant_bits(mask, b0 + tid) : 0u;
     int32_t tot;
-    int32_t m = block_exclusive_scan(c, &tot);
+    int32_t m = block_exclusive_scan(__popc(b), &tot);
     const int32_t m0 = block_offsets[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < SD_PER_THREAD; ++k) {
-        if (l0 + k >= items) break;
-        mstart[b0 + l0 + k] = m0 + m;
-        uint32_t b = bits[k];
-        while (b) {
-            sList[m++] = (uint16_t)(__builtin_ctz(b) + 8 * (l0 + k));
-            b &= b - 1;
-        }
+    if (tid < items) mstart[b0 + tid] = m0 + m;
+    while (b) {
+        sList[m++] = (uint16_t)(__builtin_ctz(b) + 8 * tid);
+        b &= b - 1;
     }
     __syncthreads();
     for (int k = tid; k < tot; k += SD_THREADS) gidx[(int64_t)m0 + k] = (int32_t)(8 * b0 + sList[k]);
@@ -122,7 +104,7 @@ __global__ __launch_bounds__(SD_THREADS) void k_emit_children(
     }
 }
 
-// The per-block child counts of tsp_subdivide_noalloc: one int32 per SD_ITEMS parents, enough
+// The per-block child counts of tsp_subdivide_noalloc: one int32 per SD_THREADS parents, enough
 // for the largest n the subdivision accepts (8n < 2^31 -> at most 2^18 blocks), 1 MiB on each
 // device. Host code reaches it only through the address hipGetSymbolAddress gives per device.
 constexpr int64_t SD_SCRATCH_WORDS = int64_t(1) << 18;
@@ -132,11 +114,11 @@ constexpr int SD_MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
 int32_t* g_scratch_ptr[SD_MAX_DEVICES] = {};
 
-// The three launches over `sums` (nb = ceil(n / SD_ITEMS) int32; every entry is written by
+// The three launches over `sums` (nb = ceil(n / SD_THREADS) int32; every entry is written by
 // k_block_counts before it is read, so nothing needs clearing).
 int subdivide_launch(const uint8_t* mask, const int32_t* coords, int64_t n, int32_t* mstart,
                      int32_t* child, int32_t* gidx, int64_t* m_out, int32_t* sums, hipStream_t s) {
-    const int64_t nb = ceil_div(n, SD_ITEMS);
+    const int64_t nb = ceil_div(n, SD_THREADS);
     if (nb > 0) {
         hipLaunchKernelGGL(k_block_counts, dim3((unsigned)nb), dim3(SD_THREADS), 0, s, mask, n, sums);
         TSP_CHECK_LAUNCH();
@@ -169,7 +151,7 @@ using namespace tsp;
 
 extern "C" size_t tsp_subdivide_workspace_bytes(int64_t n) {
     if (n < 0) return 0;
-    const int64_t nb = std::max<int64_t>(1, ceil_div(n, SD_ITEMS));
+    const int64_t nb = std::max<int64_t>(1, ceil_div(n, SD_THREADS));
     return (size_t)nb * sizeof(int32_t);
 }
 
@@ -196,10 +178,10 @@ extern "C" int tsp_subdivide_noalloc(const uint8_t* d_mask, const int32_t* d_coo
     if (int st = check_subdivide_args("tsp_subdivide_noalloc", d_mask, d_coords, n, d_mstart,
                                       d_child_coords, d_gidx, d_m))
         return st;
-    const int64_t nb = ceil_div(n, SD_ITEMS);
+    const int64_t nb = ceil_div(n, SD_THREADS);
     TSP_REQUIRE(nb <= SD_SCRATCH_WORDS, TSP_ERR_INVALID,
                 "tsp_subdivide_noalloc: n=%lld exceeds the scratch's %lld parents", (long long)n,
-                (long long)(SD_SCRATCH_WORDS * SD_ITEMS));
+                (long long)(SD_SCRATCH_WORDS * SD_THREADS));
     int dev = 0;
     TSP_CHECK_HIP(hipGetDevice(&dev));
     TSP_REQUIRE(dev >= 0 && dev < SD_MAX_DEVICES, TSP_ERR_INVALID,
