@@ -417,3 +417,25 @@ def test_library_gemm_needs_no_workspace(pkg):
     assert pick((4096, 0), (0, 0)) == 1
     assert pick((0, 7), (4096, 0), (0, 0)) == 2
     assert pick((4096, 0), (0, 3)) == -1
+
+
+# voxels, ci, co: whether every kind of call (a Morton plan, a plan of rows, no plan) measured at least as fast
+# on the small-grid conv as on the large-grid one, on 256 compute units
+SPLIT_PAYS = [(2606, 64, 64, True), (4099, 1024, 1024, True), (4300, 256, 2048, True), (8400, 512, 512, True),
+              (9000, 1024, 1024, True), (22000, 1024, 1024, True), (35001, 512, 512, True), (45000, 1024, 512, True),
+              (17000, 512, 512, False), (33500, 256, 256, False), (33500, 512, 256, False), (33500, 1024, 1024, False),
+              (45000, 256, 256, False), (45000, 512, 256, False), (66000, 256, 256, False), (80000, 256, 128, False),
+              (117343, 256, 256, False), (643361, 128, 128, False)]
+
+
+@pytest.mark.parametrize("n,ci,co,split", SPLIT_PAYS)
+def test_small_grid_conv_rule(pkg, n, ci, co, split):
+    """The conv takes one kernel for a size, with a plan or without (the sums are in one order), so the
+    small-grid one only where no kind of call is slower on it: where its units run in several rounds, a
+    plan of rows and no plan were 10-20 % slower while a Morton plan gained 2-7 %."""
+    rule = pkg.lib()["_ZN3tsp15conv_split_pickEliii"]
+    rule.argtypes, rule.restype = [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int], ctypes.c_int
+    import torch
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rule follows the device's compute units")
+    assert (rule(n, ci, co, 1) > 0) == split

@@ -74,14 +74,25 @@ int conv_split_pick(int64_t n, int ci, int co, int ncg) {
     // of units costs so much per 16-channel slice, plus a fixed part (the large-grid kernel's tiles
     // are pipelined and pay it once; a thin last round costs it 5.6 a slice, column_split_tiles).
     const int64_t big = tiles * (co % 128 == 0 ? co / 128 : co / 64);
-    const double per = co % 128 == 0 ? 9.3 : 4.6;
     int64_t whole = ceil_div(big, cus);
+    double per = co % 128 == 0 ? 9.3 : 4.6;
+    // One round of the large-grid kernel runs faster on a part of the chip: 33.5 K and 45 K 256 -> 256, a
+    // half and two thirds of a round, 137 and 146 us where a full one is 158.
+    if (whole == 1) per *= 0.84 + 0.32 * std::max(0.0, (double)big / (double)cus - 0.5);
     double base = 9.0;
     if (ncg == 1 && co % 128 == 0 && column_split_tiles(tiles, co / 128, (int)cus) > 0) {
         whole -= 1;
         base += 5.6 * (double)nkc;
     }
-    double best = 0.95 * (base + per * (double)(whole * nkc));   // (a margin: the split must be worth it)
+    const double large = base + per * (double)(whole * nkc);
+    // The units of a tile each stage its rows, and more of them on a plan of consecutive rows or without
+    // a plan, which take the same kernel. Where those rows come from L2 (features of up to 8 MiB, or the
+    // units that run together share few tiles) or are staged once a column tile, a twentieth less
+    // time is enough; elsewhere a twelfth: 33.5 K 512 -> 256, in three rounds of units of two row groups, was
+    // 243 us on a Morton plan (262 on the large-grid kernel), but 294 on rows (261) and 488 without a
+    // plan (440).
+    const bool in_l2 = n * (int64_t)ci * 2 <= ((int64_t)8 << 20);
+    double best = large;
     int pick = 0;
     const int64_t full = n / HB_M, rem = n % HB_M;
     const int64_t last = rem ? std::min<int64_t>(4, ceil_div(rem, 32)) : 0;   // row groups of the last tile
@@ -89,9 +100,11 @@ int conv_split_pick(int64_t n, int ci, int co, int ncg) {
         const int64_t units = (full * (4 / rgw) + ceil_div(last, rgw)) * (co / (64 * ncg));
         const int w = rgw * ncg;
         const int64_t rounds = ceil_div(units, cus);
-        const double slice = w == 4 ? 4.6 : w == 2 ? (rounds > 1 ? 2.45 : 2.2) : (rounds > 1 ? 1.6 : 1.45);
+        const double slice = w == 4 ? 4.6 : w == 2 ? (rounds == 1 ? 2.2 : in_l2 ? 2.255 : 2.45) : (rounds > 1 ? 1.6 : 1.45);
         const double cost = 4.0 + (double)rounds * (6.0 + slice * (double)nkc);
-        if (cost < best) {
+        const int64_t share = (4 / rgw) * (co / (64 * ncg));   // units of a tile
+        const bool near = w == 4 || share >= 64 || (share >= 32 && whole == 1);
+        if (cost < best && cost < (in_l2 ? 0.955 : near ? 0.95 : 0.92) * large) {
             best = cost;
             pick = rgw;
         }
