@@ -1,10 +1,11 @@
-"""GPU parity of the C2S block on an octant plan (csrc/plan.hip octant_plan_build): conv1 over each
-octant's kept parents only.
+"""GPU parity of the C2S block with an octant plan (csrc/plan.hip octant_plan_build): conv1 over each
+octant's kept parents only, where the device finds that it pays.
 
 The cases sit where the plan can go wrong: octants kept by half, a quarter (tiles of fewer than 512
-parents) and three quarters of the parents; octants with very different totals, one with none; plan
-tiles of consecutive rows instead of the Morton order; scattered voxels, whose octant tiles exceed
-the staged rows; and both conv kernels (large grid, small grid)."""
+parents) and three quarters of the parents; both conv kernels (large grid, small grid); and where it
+is built and not run: octants with very different totals, one with none; plan tiles of consecutive
+rows and scattered voxels, whose octant tiles exceed the staged rows; a single round of units.
+test_gpu_octant_plan_corners.py reads which of the two plans was run."""
 from __future__ import annotations
 
 import numpy as np

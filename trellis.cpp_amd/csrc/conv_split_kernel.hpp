@@ -17,11 +17,12 @@
 // Measured (one MI355X, us a conv, against the large-grid kernel, whose 512-voxel x 128-channel
 // units are too few here): 2.6 K voxels 64 -> 64 f16 26 -> 13; 1.2 K 512 -> 512 253 -> 49;
 // 4.1 K 1024 -> 1024 508 -> 266; 15 K 128 -> 128 70 -> 21; 35 K 512 -> 512 (1.08 rounds there)
-// 499 -> 418; the C2S block 256 -> 128 on 2.6 K 235 -> 80. What bounds it: a slice of a 1-row-group
-// unit takes 1.3 us for 0.67 us of MFMA issue; without the slice pieces it runs 12-20 % faster,
-// with every weight read from one address 10 %, and the rest is the fixed 5-6 us of a unit (plan,
-// first slice, the partial sums) and the last round of units. An issue priority alternating between
-// the waves, which the large-grid kernel takes, costs 3-7 % here.
+// 499 -> 418; the C2S block 256 -> 128 on 2.6 K 235 -> 80. What bounds it: the latency of a slice (rows,
+// weights, the barrier) and the CUs left idle. 4.1 K 1024 -> 1024, 144 units: the matrix cores are busy 31 %
+// of the chip's cycles, 56 % of those of the CUs in use, and the waves wait 39 % of theirs; the rest
+// is a unit's fixed 5-6 us (plan, first slice, the partial sums). Left out, the slice pieces give
+// 12-20 %, the spread of the weights' addresses 10 %. An issue priority alternating between the waves,
+// which the large-grid kernel takes, costs 3-7 % here.
 #include "conv_halo_kernel.hpp"
 
 namespace tsp {
