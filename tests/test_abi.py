@@ -399,24 +399,46 @@ def test_float32_vectors(pkg, call):
 
 
 def test_library_gemm_needs_no_workspace(pkg):
-    """The linear layers call the GEMM library without a workspace: of the heuristic's results only one
-    whose state is success and that asks for none may run."""
+    """The linear layers call the GEMM library without a workspace: the heuristic's first result runs only
+    where its state is success and it asks for none."""
     class Result(ctypes.Structure):   # hipblasLtMatmulHeuristicResult_t
         _fields_ = [("algo", ctypes.c_uint8 * 24), ("workspace", ctypes.c_size_t), ("state", ctypes.c_int),
                     ("waves", ctypes.c_float), ("reserved", ctypes.c_int * 4)]
     usable = pkg.lib()["_ZN3tsp13blaslt_usableEPK33_hipblasLtMatmulHeuristicResult_ti"]
-    usable.restype = ctypes.c_int
+    usable.restype = ctypes.c_bool
 
-    def pick(*results):
-        a = (Result * max(1, len(results)))()
-        for k, (ws, state) in enumerate(results):
-            a[k].workspace, a[k].state = ws, state
-        return usable(a, len(results))
-    assert pick() == -1
-    assert pick((0, 0), (0, 0)) == 0
-    assert pick((4096, 0), (0, 0)) == 1
-    assert pick((0, 7), (4096, 0), (0, 0)) == 2
-    assert pick((4096, 0), (0, 3)) == -1
+    def one(ws, state, count=1):
+        r = Result()
+        r.workspace, r.state = ws, state
+        return usable(ctypes.byref(r), count)
+    assert one(0, 0) and not one(4096, 0) and not one(0, 7) and not one(0, 0, count=0)
+
+
+@pytest.mark.parametrize("n", [1, 255, 4096, 8200, 16384, 16385, 35001, 70000, 262144])
+def test_library_gemm_pieces(pkg, n):
+    """Rows are cut into pieces whose algorithm is usable, the largest first, and refused where one has
+    none; every row is in one piece."""
+    Usable = ctypes.CFUNCTYPE(ctypes.c_bool, ctypes.c_int64, ctypes.c_void_p)
+    piece = pkg.lib()["_ZN3tsp12blaslt_pieceElPFblPvES0_"]
+    piece.argtypes, piece.restype = [ctypes.c_int64, Usable, ctypes.c_void_p], ctypes.c_int64
+
+    def cut(rule):
+        asked, pieces, left = [], [], n
+        rule_c = Usable(lambda k, _: (asked.append(k), rule(k))[1])
+        while left:
+            p = piece(left, rule_c, None)
+            if p == 0:
+                return None, asked
+            assert 0 < p <= left and rule(p)
+            pieces.append(p)
+            left -= p
+        return pieces, asked
+    assert cut(lambda k: True) == ([n], [n])
+    assert cut(lambda k: False)[0] is None
+    for rule in (lambda k: k != n, lambda k: k % 8192 == 0 or k < 9000, lambda k: k <= 20000):
+        pieces, asked = cut(rule)
+        assert sum(pieces) == n if pieces else n == 1
+        assert len(set(asked)) < 80   # (each shape is asked of the library once)
 
 
 # voxels, ci, co: whether every kind of call (a Morton plan, a plan of rows, no plan) measured at least as fast

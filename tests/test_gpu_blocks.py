@@ -84,8 +84,8 @@ def test_linear_ex(gpu_lib, orc, n, ci, co):
                                                   (134000, 256, 64, "none", True), (134000, 512, 8, "none", False)])
 @pytest.mark.parametrize("key", ["bfloat16", "float16"])
 def test_linear_ex_without_workspace(gpu_lib, n, ci, co, act, residual, key):
-    """Shapes for which a build of the GEMM library lists first a kernel that needs a workspace, or (70 K of
-    4096 -> 1024) none that does not: sampled rows, of both halves, against fp64."""
+    """Shapes for which a build of the GEMM library chooses a kernel that needs a workspace, so that their
+    rows are cut: sampled rows, around a cut at a multiple of 4096 too, against fp64."""
     import torch
     print(f"[linear] no workspace n={n} {ci}->{co} {act} residual={residual} {key}", flush=True)
     dt = getattr(torch, key)
@@ -95,7 +95,8 @@ def test_linear_ex_without_workspace(gpu_lib, n, ci, co, act, residual, key):
     b = torch.randn(co, generator=g, device="cuda")
     r = torch.randn((n, co), generator=g, device="cuda") if residual else None
     out = gpu_lib.linear_ex(x, w, b, act=act, residual=r, out_dtype=torch.float32 if act == "none" else dt)
-    rows = torch.cat([torch.arange(300), torch.arange(n // 2 - 300, n // 2 + 300), torch.arange(n - 300, n)]).cuda()
+    rows = torch.cat([torch.arange(300), torch.arange(n // 2 - 300, n // 2 + 300),
+                      torch.arange((n - 1) // 4096 * 4096 - 200, n)[:500], torch.arange(n - 300, n)]).cuda()
     ref = x[rows].cpu().double() @ w.cpu().double().t() + b.cpu().double()
     if act == "silu":
         ref = ref / (1 + torch.exp(-ref))

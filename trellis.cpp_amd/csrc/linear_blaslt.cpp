@@ -7,14 +7,16 @@
 // Algorithms come from hipBLASLt's heuristic with no workspace, cached per shape and device. Some builds
 // of the library return kernels that need one all the same (stream-K kernels, whose partial sums then
 // go to a null pointer: illegal accesses at 8.2 K rows of 512 -> 2048, 70 K of 256 -> 1024, while 35 K
-// of 512 -> 2048 ran), so only results that ask for none are used, and where there is none among
-// them, the call is cut into fewer rows.
+// of 512 -> 2048 ran). So only a first choice that asks for none is used; where it asks, the rows are cut
+// where the choice for the larger piece does not (asked for more results, the heuristic takes 25 ms a
+// shape instead of 0.1).
 #include <hipblaslt/hipblaslt.h>
 
 #include <map>
 #include <algorithm>
 #include <mutex>
 #include <tuple>
+#include <vector>
 
 #include "conv_internal.hpp"
 
@@ -61,13 +63,20 @@ struct Gemm {
 
 }  // namespace
 
-// The first of the heuristic's results that may run without a workspace, -1 when there is none: a
-// result's other fields hold only with state SUCCESS, and its kernel writes partial sums to the
-// workspace it asks for.
-int blaslt_usable(const hipblasLtMatmulHeuristicResult_t* results, int count) {
-    for (int k = 0; k < count; ++k)
-        if (results[k].state == HIPBLAS_STATUS_SUCCESS && results[k].workspaceSize == 0) return k;
-    return -1;
+// Whether the heuristic's first result may run without a workspace: its other fields hold only with
+// state SUCCESS, and its kernel writes partial sums to the workspace it asks for.
+bool blaslt_usable(const hipblasLtMatmulHeuristicResult_t* results, int count) {
+    return count > 0 && results[0].state == HIPBLAS_STATUS_SUCCESS && results[0].workspaceSize == 0;
+}
+
+// The rows of the next library call of n: all of them where usable(n), else the largest usable multiple
+// of 4096 below (of 256 up to 16384 rows, of 16 up to 256), 0 where there is none.
+int64_t blaslt_piece(int64_t n, bool (*usable)(int64_t, void*), void* arg) {
+    if (usable(n, arg)) return n;
+    const int64_t step = n > 16384 ? 4096 : n > 256 ? 256 : 16;
+    for (int64_t c = (n - 1) / step * step; c > 0; c -= step)
+        if (usable(c, arg)) return c;
+    return 0;
 }
 
 bool blaslt_eligible(int x_dtype, int weight_dtype, int out_dtype, int ci, int co, const void* x,
@@ -94,35 +103,44 @@ int64_t blaslt_rows_per_call(int ci, int co, int xdt, int odt, bool residual) {
 }
 
 // Row chunks of blaslt_rows_per_call rows: one library call never addresses 2^31 bytes or more
-// in an operand (the composite blocks already bound their hidden layers to 1 GiB). Chunks for which the
-// library has no usable algorithm are halved down to 4096 rows; nothing is launched before every
-// chunk has one.
+// in an operand (the composite blocks already bound their hidden layers to 1 GiB), cut further where
+// the library's algorithm would need a workspace (blaslt_piece). Nothing is launched before every
+// piece has an algorithm.
 int blaslt_linear(const void* x, int xdt, int64_t n, int ci, const void* w, const float* bias,
                   int co, int act, const float* residual, void* out, int odt, hipStream_t s) {
-    if (n <= 0) return TSP_OK;
-    int64_t rows = std::min(n, blaslt_rows_per_call(ci, co, xdt, odt, residual != nullptr));
+    const int64_t rows = blaslt_rows_per_call(ci, co, xdt, odt, residual != nullptr);
     TSP_REQUIRE(rows > 0, TSP_ERR_UNSUPPORTED, "linear: a row of ci=%d co=%d spans 2 GiB", ci, co);
-    auto each = [&](bool launch) {
-        for (int64_t r0 = 0; r0 < n; r0 += rows) {
-            const int64_t nr = std::min(rows, n - r0);
-            const int st = blaslt_linear_rows(static_cast<const char*>(x) + r0 * ci * (int64_t)dtype_size(xdt), xdt, nr,
-                                              ci, w, bias, co, act, residual ? residual + r0 * co : nullptr,
-                                              static_cast<char*>(out) + r0 * co * (int64_t)dtype_size(odt), odt, s, launch);
-            if (st != TSP_OK) return st;
-            if (!launch && r0 == 0 && n % rows && n > 2 * rows) r0 = n / rows * rows - rows;   // (then the last, shorter one)
-        }
-        return (int)TSP_OK;
+    auto call = [&](int64_t r0, int64_t nr, bool launch) {
+        return blaslt_linear_rows(static_cast<const char*>(x) + r0 * ci * (int64_t)dtype_size(xdt), xdt, nr, ci, w, bias, co,
+                                  act, residual ? residual + r0 * co : nullptr,
+                                  static_cast<char*>(out) + r0 * co * (int64_t)dtype_size(odt), odt, s, launch);
     };
-    for (;;) {
-        const bool one = rows >= n;
-        const int st = each(one);
-        if (st == TSP_OK) {
-            clear_error();
-            return one ? st : each(true);
-        }
-        if (st != TSP_ERR_UNSUPPORTED || rows <= 4096) return st;
-        rows = ceil_div(rows, 512) * 256;
+    if (n <= rows) {
+        const int st = n > 0 ? call(0, n, true) : TSP_OK;
+        if (st != TSP_ERR_UNSUPPORTED) return st;
     }
+    std::vector<int64_t> pieces;
+    int st = TSP_OK;
+    auto usable = [&](int64_t nr) {
+        const int q = call(0, nr, false);
+        if (q != TSP_OK) st = q;
+        return q == TSP_OK;
+    };
+    using Usable = decltype(usable);
+    for (int64_t r0 = 0; r0 < n;) {
+        const int64_t p = blaslt_piece(std::min(rows, n - r0), [](int64_t nr, void* u) { return (*static_cast<Usable*>(u))(nr); },
+                                       &usable);
+        if (p == 0) return st;
+        pieces.push_back(p);
+        r0 += p;
+    }
+    clear_error();
+    int64_t r0 = 0;
+    for (const int64_t p : pieces) {
+        if ((st = call(r0, p, true)) != TSP_OK) return st;
+        r0 += p;
+    }
+    return TSP_OK;
 }
 
 static int blaslt_linear_rows(const void* x, int xdt, int64_t n, int ci, const void* w, const float* bias,
@@ -166,20 +184,14 @@ static int blaslt_linear_rows(const void* x, int xdt, int64_t n, int ci, const v
         AlgoEntry e;
         hipblasLtMatmulPreference_t pref = nullptr;
         uint64_t ws = 0;
-        // the heuristic's first choice, or the first that is usable of many
-        hipblasLtMatmulHeuristicResult_t res[64]{};
-        int count = 0, pick = -1;
+        hipblasLtMatmulHeuristicResult_t res[1]{};
+        int count = 0;
         if (hipblasLtMatmulPreferenceCreate(&pref) == HIPBLAS_STATUS_SUCCESS &&
-            hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws)) == HIPBLAS_STATUS_SUCCESS) {
-            for (int want : {1, 64}) {
-                if (hipblasLtMatmulAlgoGetHeuristic(h, g.desc, g.a, g.b, g.c, g.d, pref, want, res, &count) == HIPBLAS_STATUS_SUCCESS)
-                    pick = blaslt_usable(res, std::min(count, want));
-                if (pick >= 0) break;
-            }
-        }
-        if (pick >= 0) {
+            hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws)) == HIPBLAS_STATUS_SUCCESS &&
+            hipblasLtMatmulAlgoGetHeuristic(h, g.desc, g.a, g.b, g.c, g.d, pref, 1, res, &count) == HIPBLAS_STATUS_SUCCESS &&
+            blaslt_usable(res, count)) {
             e.ok = true;
-            e.algo = res[pick].algo;
+            e.algo = res[0].algo;
         }
         if (pref) hipblasLtMatmulPreferenceDestroy(pref);
         it = g_algos.emplace(key, e).first;
