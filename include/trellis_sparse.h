@@ -287,7 +287,8 @@ int tsp_linear_ex(const void* d_x, int x_dtype, int64_t n, int ci, const void* d
 /* Rows of x that tsp_linear and tsp_linear_ex hand hipBLASLt per library call: they cut n into
  * chunks of this many rows so that no operand of one call (x, out, residual) spans 2^31 bytes or
  * more (the counterpart of the reference's mul_mat_rows, sparse.cpp:41-59, which cuts at
- * 1,000,000 rows for a Vulkan grid limit). A multiple of 256 where 256 rows fit; 0 for invalid
+ * 1,000,000 rows for a Vulkan grid limit), and a chunk for which the library's algorithm would
+ * need a workspace into smaller ones, so this is the most that one call gets. A multiple of 256 where 256 rows fit; 0 for invalid
  * arguments or a row of 2 GiB. Host arithmetic only (no device call). */
 int64_t tsp_linear_rows_per_call(int ci, int co, int x_dtype, int out_dtype, int has_residual);
 
