@@ -22,15 +22,19 @@ def _without_plan(n, m, cin, cout):
             + _al(16 * -(-n // 512)))
 
 
-def _block(tsp, shells, n, cin, cout, keep, key="bf16", seed=0):
-    """A C2S block with device tensors: n parents of a shell, octant o kept with probability keep[o]."""
+def _block(tsp, shells, n, cin, cout, keep, key="bf16", seed=0, counts=None):
+    """A C2S block with device tensors: n parents of a shell, octant o kept with probability keep[o], or by
+    exactly counts[o] of them."""
     import torch
     dt = torch.bfloat16 if key == "bf16" else torch.float16
     rng = np.random.default_rng(n + cin + seed)
     coords = shells.sphere_shell(96, 48.0, 34.0, 36.4 if n > 12000 else 35.6)
     assert len(coords) >= n
     c = torch.from_numpy(np.ascontiguousarray(coords[:n], np.int32)).cuda()
-    mask = torch.from_numpy((rng.random((n, 8)) < np.asarray(keep)).astype(np.uint8).reshape(-1)).cuda()
+    mask = (rng.random((n, 8)) < np.asarray(keep)).astype(np.uint8)
+    if counts is not None:
+        mask = np.stack([rng.permutation(n) < k for k in counts], 1).astype(np.uint8)
+    mask = torch.from_numpy(mask.reshape(-1)).cuda()
     g = torch.Generator(device="cuda")
     g.manual_seed(n + seed)
     rand = lambda shape, std, d: (torch.randn(shape, generator=g, device="cuda") * std).to(d)
@@ -216,3 +220,37 @@ def test_values_not_finite(gpu_lib, shells, n, cin, cout, bad):
     assert bool(want.isnan().any()) and torch.equal(got.isnan(), want.isnan())
     assert torch.equal(got.nan_to_num(0.0), want.nan_to_num(0.0))
 
+
+def test_captured(gpu_lib, shells):
+    """The block in a captured graph, replayed with an even mask and with one that keeps two octants whole
+    (the same number of children): each replay decides for its own mask, and matches the eager block."""
+    import torch
+    print("[octant plan] captured", flush=True)
+    n, cin, cout = 24000, 256, 128
+    even = _block(gpu_lib, shells, n, cin, cout, [0.5] * 8, counts=[n // 2] * 8)
+    full_two = _block(gpu_lib, shells, n, cin, cout, [0.5] * 8, counts=[n] * 2 + [n // 3] * 6)
+    assert even["m"] == full_two["m"]
+    size, less = _bytes(gpu_lib, even), _without_plan(n, even["m"], cin, cout)
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+    want, took = {}, {}
+    for name, b in (("even", even), ("two", full_two)):
+        b["p"] = even["p"]
+        st, want[name] = _run(gpu_lib, b, ws, size)
+        assert st == 0
+        took[name] = int(ws[less:less + 4].view(torch.int32)[0])
+    assert took["even"] == 1
+    live = {k: even[k].clone() for k in ("x", "nbr", "plan", "mask", "gidx", "mstart", "cnbr", "cplan")}
+    b = {**even, **live}
+    out = torch.empty((b["m"], cout), device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert _part(gpu_lib, b, ws, size, out, 3) == 0
+    for name, src in (("even", even), ("two", full_two), ("two", full_two), ("even", even)):
+        for k, t in live.items():
+            t.copy_(src[k])
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert int(ws[less:less + 4].view(torch.int32)[0]) == took[name]
+        assert torch.equal(out, want[name])
