@@ -1,5 +1,5 @@
 """The C2S block's octant plan (csrc/plan.hip) where it is not the usual call: a workspace without
-room for it; masks that keep some octants far more often than others; the
+room for it, or not aligned; masks that keep some octants far more often than others; the
 block in parts; weights and a row 0 that are not finite."""
 from __future__ import annotations
 
@@ -61,7 +61,7 @@ def _weights(tsp, p):
 def _run(tsp, b, ws, ws_bytes):
     """tsp_c2s on the workspace's first ws_bytes -> (status, out)."""
     import torch
-    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None
     out = torch.full((b["m"], b["cout"]), float("nan"), device="cuda")
     st = tsp.lib().tsp_c2s(ptr(b["x"]), b["n"], b["cin"], ptr(b["nbr"]), ptr(b["plan"]), ptr(b["mask"]), ptr(b["mstart"]),
                            ptr(b["gidx"]), b["m"], b["cout"], ptr(b["cnbr"]), ptr(b["cplan"]),
@@ -99,6 +99,29 @@ def test_workspace_without_the_plan(gpu_lib, shells, n, cin, cout):
     assert _bytes(gpu_lib, b, 8 * n) == _without_plan(n, 8 * n, cin, cout)
     st, got = _run(gpu_lib, b, ws, min(full, _bytes(gpu_lib, b, 8 * n)))
     assert st == 0 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n,cin,cout", [(14001, 256, 128), (24000, 256, 128)])
+def test_workspace_not_aligned(gpu_lib, shells, n, cin, cout):
+    """A workspace 8 bytes off 16 runs conv1 without an octant plan: with no child plan the block is the
+    aligned one's up to the order of conv2's sums (at most 2 K eps sum|w h|, |h| of rms about 0.6 after
+    LN + SiLU and |w_o| about 1); with one it is refused, as conv2 on the matrix cores needs 16 bytes."""
+    import torch
+    print(f"[octant plan] unaligned workspace n={n} {cin}->{cout}", flush=True)
+    b = _block(gpu_lib, shells, n, cin, cout, [0.5] * 8)
+    size = _bytes(gpu_lib, b)
+    assert _without_plan(n, b["m"], cin, cout) < size, "the case is meant to take an octant plan"
+    ws = torch.full((size + 16,), 0xA5, dtype=torch.uint8, device="cuda")
+    assert _run(gpu_lib, b, ws[8:], size)[0] == 1
+    b = {**b, "cplan": None}
+    st, want = _run(gpu_lib, b, ws, size)
+    assert st == 0
+    ws.fill_(0xA5)
+    st, got = _run(gpu_lib, b, ws[8:], size)
+    k = 27 * cout
+    assert st == 0
+    torch.testing.assert_close(got, want, rtol=0, atol=2 * k * 2.0 ** -24 * k ** 0.5)
+    assert bool((ws[:8] == 0xA5).all()) and bool((ws[8 + size:] == 0xA5).all())
 
 
 # keep probabilities of the octants, and whether the plan then pays: only where its fullest octant has
